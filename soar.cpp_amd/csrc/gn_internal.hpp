@@ -257,6 +257,20 @@ hipError_t launch_pw_conv(const PwArgs& a, int64_t N, int64_t C_in, int64_t C_ou
                           int64_t HW, int64_t chunk, double2* part, bool accumulate,
                           int64_t small, float* kz_ws, int kz_max, hipStream_t s,
                           const char* name = nullptr, bool wt = false);
+// The block-tiled convolution of wide layers (pw_gemm.hip): M output rows,
+// K input rows; `trans`: weights [K][M].  chunk as for launch_pw_conv.
+bool pw_gemm_use(int64_t N, int64_t K, int64_t M, int64_t HW);
+hipError_t launch_pw_gemm(const PwArgs& a, int64_t N, int64_t K, int64_t M, int64_t HW,
+                          int64_t chunk, double2* part, bool accumulate, bool trans,
+                          hipStream_t s);
+// Its weight gradient: partials of every pixel chunk of every sample,
+// part_w[chunk][C_out][C_in] and (nullable) part_b[chunk][C_out].
+bool pw_gemm_wgrad_use(int64_t N, int64_t C_in, int64_t C_out, int64_t HW);
+int64_t pw_gemm_wgrad_chunk(int64_t N, int64_t C_in, int64_t C_out, int64_t HW);
+hipError_t launch_pw_gemm_wgrad(const float* dz, const float* x, float* part_w, float* part_b,
+                                int64_t N, int64_t C_in, int64_t C_out, int64_t HW, int64_t chunk,
+                                hipStream_t s);
+
 // Cross-block split-K of the MFMA convolution (kz = 1: not used).
 struct PwKz {
     int kz = 1;
@@ -292,6 +306,7 @@ struct PwBwdPlan {
     int64_t chunk_b = 0, cpp_b = 0, Gb = 0;  // their chunks: pixels, per plane, partials
     size_t wt_bytes = 0, pw_bytes = 0, pb_bytes = 0;
     int64_t chunk_dx = 0;  // pixels per wave of dx = W^T dz
+    bool gemm_dw = false;  // dW on the block-tiled kernel (pw_gemm.hip)
     int kz_dx = 1;         // its cross-block split-K (pw_kz_plan)
     size_t kz_bytes = 0;   // and the slices' bytes, after the partials
 };

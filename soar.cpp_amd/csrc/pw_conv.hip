@@ -1656,7 +1656,7 @@ bool pw_use_small_wgrad(int64_t N, int64_t C_in, int64_t C_out, int64_t HW, int6
 // us), ties at 2^26 and loses above (512 -> 256 at 1024: 34 vs 28 us; 128
 // -> 256 at 4096: 35 vs 16 us).
 bool pw_use_small(int64_t N, int64_t M, int64_t K, int64_t HW, int64_t small) {
-    return small > 0 && pw_small_fits(N, M, K, HW) &&
+    return small > 0 && pw_small_fits(N, M, K, HW) && !pw_gemm_use(N, K, M, HW) &&
            (double)N * (double)M * (double)K * (double)HW <= (double)small;
 }
 
@@ -1853,6 +1853,12 @@ hipError_t launch_pw_conv(const PwArgs& a, int64_t N, int64_t C_in, int64_t C_ou
     if (!part && pw_use_small(N, C_out, C_in, HW, small))
         return launch_pw_small(a.x, a.w, a.bias, a.z, N, C_in, C_out, HW, false, accumulate, s,
                                name ? name : "pw_conv_small");
+    if (pw_gemm_use(N, C_in, C_out, HW)) {
+        const int tok = prof_begin(s, name ? name : (part ? "pw_conv_gn_stats" : "pw_conv"));
+        const hipError_t e = launch_pw_gemm(a, N, C_in, C_out, HW, chunk, part, accumulate, wt, s);
+        prof_end(s, tok);
+        return e;
+    }
     if (kz_ws && part) {
         const PwKz kp = pw_kz_plan(N, C_in, C_out, HW, chunk, kz_max);
         if (kp.kz > 1) {
@@ -1975,6 +1981,13 @@ PwBwdPlan make_pw_bwd_plan(int64_t N, int64_t C_in, int64_t C_out, int64_t HW,
     p.cpp_b = (HW + p.chunk_b - 1) / p.chunk_b;
     p.Gb = N * p.cpp_b;
     auto al = [](size_t b) { return (b + 255) & ~(size_t)255; };
+    p.gemm_dw = pw_gemm_wgrad_use(N, C_in, C_out, HW);
+    if (p.gemm_dw) {  // one partial per chunk and sample
+        p.chunk_b = pw_gemm_wgrad_chunk(N, C_in, C_out, HW);
+        p.cpp_b = (HW + p.chunk_b - 1) / p.chunk_b;
+        p.Gb = N * p.cpp_b;
+        p.G = std::max(p.G, p.Gb);
+    }
     p.wt_bytes = al(sizeof(float) * (size_t)(C_in * C_out));
     p.pw_bytes = al(sizeof(float) * (size_t)(p.G * C_out * C_in));
     p.pb_bytes = al(sizeof(float) * (size_t)(p.G * C_out));
@@ -2025,7 +2038,7 @@ hipError_t launch_pw_backward(const PwBwdPlan& p, const PwBwdArgs& a, int64_t N,
         // loads); large grids transpose W into the workspace first.
         const int64_t cpp = (HW + p.chunk_dx - 1) / p.chunk_dx;
         const int64_t R = (C_in + kRowTile - 1) / kRowTile;
-        const bool in_place = N * cpp * R < kKzTiles;
+        const bool in_place = N * cpp * R < kKzTiles || pw_gemm_use(N, C_out, C_in, HW);
         if (!in_place) {
             const int64_t E = C_in * C_out;
             int tok = prof_begin(s, "pw_transpose");
@@ -2055,11 +2068,16 @@ hipError_t launch_pw_backward(const PwBwdPlan& p, const PwBwdArgs& a, int64_t N,
                           ((uintptr_t)a.x % 16 == 0);
         const dim3 grid((unsigned)(p.tiles_co * p.tiles_ci), (unsigned)p.Gb);
         int tok = prof_begin(s, "pw_conv_wgrad");
+        if (p.gemm_dw) {
+            const hipError_t e = launch_pw_gemm_wgrad(a.dz, a.x, part_w, a.db ? part_b : nullptr,
+                                                      N, C_in, C_out, HW, p.chunk_b, s);
+            if (e != hipSuccess) return e;
+        }
         auto launch = [&](auto F, auto M2, auto N2, auto W) {
             k_pw_wgrad<F(), M2() ? 2 : 1, N2() ? 2 : 1, W()><<<grid, 64 * W(), 0, s>>>(
                 a.dz, a.x, part_w, part_b, C_in, C_out, HW, p.chunk_b, p.cpp_b, p.tiles_ci);
         };
-        bsel(fast, [&](auto F) {
+        if (!p.gemm_dw) bsel(fast, [&](auto F) {
             bsel(p.tm == 2, [&](auto M2) {
                 bsel(p.tn == 2, [&](auto N2) {
                     switch (p.wpb) {
