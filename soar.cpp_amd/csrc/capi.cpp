@@ -357,7 +357,6 @@ SOAR_API int soar_gn_silu_forward(const float* x, const float* gamma, const floa
     Plan p;
     if (!soar::gn::make_plan(N, C, HW, G, t, &p))
         return fail(SOAR_EINVAL, "shape is too large for one launch grid");
-    p.vec4 = p.vec4 && aligned16(x) && aligned16(y);
     if ((rc = check_ws(p, workspace, workspace_bytes))) return rc;
     soar::gn::FwdArgs a{x, gamma, beta, y, mean, rstd, mean_lo, eps, flags, workspace};
     hipError_t e = soar::gn::launch_forward(p, t, a, static_cast<hipStream_t>(stream));
@@ -421,7 +420,6 @@ int gn_backward(const float* dy, const float* x, const float* gamma, const float
     Plan p;
     if (!soar::gn::make_plan(N, C, HW, G, t, &p))
         return fail(SOAR_EINVAL, "shape is too large for one launch grid");
-    p.vec4 = p.vec4 && aligned16(x) && aligned16(dy) && aligned16(dx);
     if (ws_scratch) {
         // the library's static scratch: its size is known, and it is not a
         // hipMalloc allocation to look up
@@ -594,7 +592,6 @@ int pw_conv_gn_forward(const float* x, const float* weight, const float* bias,
     Plan p;
     if (!soar::gn::make_pw_plan(N, C_out, HW, G, t, &p) || !pw_grid_fits(N, HW, p.chunk))
         return fail(SOAR_EINVAL, "shape is too large for one launch grid");
-    p.vec4 = p.vec4 && aligned16(z) && aligned16(y);
     if ((rc = check_ws(p, workspace, workspace_bytes))) return rc;
     const hipStream_t s = static_cast<hipStream_t>(stream);
     soar::gn::PwArgs pa{x, weight, bias, z};
@@ -603,7 +600,6 @@ int pw_conv_gn_forward(const float* x, const float* weight, const float* bias,
         soar::gn::make_plan(N, C_out, HW, G, t, &q)) {
         // Small planes: the SIMT convolution (no statistics epilogue), then
         // the GroupNorm forward over z with its own plan.
-        q.vec4 = q.vec4 && aligned16(z) && aligned16(y) && (!residual || aligned16(residual));
         if ((rc = check_ws(q, workspace, workspace_bytes))) return rc;
         hipError_t e = soar::gn::launch_pw_conv(pa, N, C_in, C_out, HW, p.chunk, nullptr, false,
                                                 t.pw_small, nullptr, 1, s);
@@ -644,7 +640,6 @@ int pw_conv_gn_forward(const float* x, const float* weight, const float* bias,
     if (in_apply) {
         a.flags |= SOAR_GN_RESIDUAL;
         a.res = residual;
-        if (!aligned16(residual)) p.vec4 = false;
     }
     e = soar::gn::launch_forward_from_partials(p, t, a, s);
     if (e != hipSuccess) return hip_fail(e, "GroupNorm apply launch");
@@ -902,7 +897,6 @@ SOAR_API int soar_pw_cba_backward(const float* dy, const float* z, const float* 
                         workspace_bytes, L.fused_bytes);
         if ((rc = check_dev(workspace, L.fused_bytes, "workspace"))) return rc;
         Plan gp = L.gp;
-        gp.vec4 = gp.vec4 && aligned16(z) && aligned16(dy);
         const unsigned gflags = flags & SOAR_GN_SILU;
         soar::gn::BwdArgs a{dy, z, gamma, beta, mean, rstd, mean_lo, nullptr, dgamma, dbeta,
                             gflags, workspace};
@@ -1009,7 +1003,6 @@ SOAR_API int soar_dw_conv_gn_silu_forward(const float* x, const float* weight, c
     DwGnLayout L;
     if (!dw_gn_layout(sh, G, t, &L))
         return fail(SOAR_EINVAL, "shape is too large for one launch grid");
-    L.p.vec4 = L.p.vec4 && aligned16(z) && aligned16(y);
     if ((rc = check_ws(L.p, workspace, workspace_bytes))) return rc;
     if (workspace_bytes < L.gn_bytes + L.part_bytes)
         return fail(SOAR_EINVAL, "workspace of %zu bytes is smaller than the %zu this call needs",
@@ -1186,7 +1179,6 @@ SOAR_API int soar_dw_cba_backward(const float* dy, const float* z, const float* 
                         workspace_bytes, L.fused_bytes);
         if ((rc = check_dev(workspace, L.fused_bytes, "workspace"))) return rc;
         Plan gp = L.gp;
-        gp.vec4 = gp.vec4 && aligned16(z) && aligned16(dy);
         const unsigned gflags = flags & SOAR_GN_SILU;
         soar::gn::BwdArgs a{dy, z, gamma, beta, mean, rstd, mean_lo, nullptr, dgamma, dbeta,
                             gflags, workspace};

@@ -31,7 +31,6 @@ struct Plan {
     int64_t blocks2 = 0;     // so may cut the planes differently
     int64_t upb_fwd = 0;     // units per forward batch
     int64_t upb_bwd = 0;     // units per backward batch
-    bool vec4 = false;       // float4 path (HW % 4 == 0 and 16-byte pointers)
     int loads = 4;           // 128-bit loads in flight per thread, first passes
     bool ntl1 = false;       // non-temporal loads in the first passes ...
     int64_t nt_tail = 0;     // ... except for their last this many bytes read
