@@ -103,7 +103,8 @@ PREDICT_CONFIGS = {
 # step, summed over its launches (a kernel runs once per unit batch)
 PASSES = {"gn_stats_partial": 1, "gn_silu_apply": 2, "gn_silu_bwd_reduce": 2,
           "gn_silu_bwd_dx": 3, "gn_stats_finish": 0, "gn_bwd_finish": 0,
-          "gn_param_finish": 0}
+          "gn_param_finish": 0, "gn_silu_team_fwd": 2, "gn_team_fwd": 2,
+          "gn_silu_team_bwd": 3, "gn_team_bwd": 3}
 
 
 def parse():

@@ -601,6 +601,11 @@ SOAR_API int soar_prof_summary(char* buf, size_t buflen);
                                 /* last with cached loads (the second    */
                                 /* pass walks in reverse and reads them  */
                                 /* first, from the MALL)                 */
+#define SOAR_TUNE_TEAM_WAIT_US 20 /* GroupNorm of large units in one pass: */
+                                /* microseconds a block waits for the    */
+                                /* sums of its unit's other blocks       */
+                                /* before it computes the missing ones   */
+                                /* (-1 = two passes instead)             */
 SOAR_API int soar_gn_tune(int key, int64_t value);
 SOAR_API int64_t soar_gn_tune_get(int key);
 

@@ -1591,6 +1591,11 @@ SOAR_API int soar_gn_tune(int key, int64_t value) {
                 return fail(SOAR_EINVAL, "nt_tail_mb must be in [0, 2^20]");
             g_tune.nt_tail_mb = value;
             return ok();
+        case SOAR_TUNE_TEAM_WAIT_US:
+            if (value < -1 || value > 1000000)
+                return fail(SOAR_EINVAL, "team_wait_us must be in [-1, 10^6]");
+            g_tune.team_wait_us = value;
+            return ok();
         default:
             return fail(SOAR_EINVAL, "unknown tuning key %d", key);
     }
@@ -1616,6 +1621,7 @@ SOAR_API int64_t soar_gn_tune_get(int key) {
         case SOAR_TUNE_PW_WG_TARGET: return g_tune.pw_wg_target;
         case SOAR_TUNE_PW_CBA_MIN: return g_tune.pw_cba_min;
         case SOAR_TUNE_PW_CBA_BLOCKS: return g_tune.pw_cba_blocks;
+        case SOAR_TUNE_TEAM_WAIT_US: return g_tune.team_wait_us;
         case SOAR_TUNE_DW_CBA_MIN: return g_tune.dw_cba_min;
         case SOAR_TUNE_NT_TAIL_MB: return g_tune.nt_tail_mb;
         default: return -1;

@@ -1630,6 +1630,12 @@ hipError_t launch_forward(const Plan& p, const Tuning& t, const FwdArgs& a, hipS
         prof_end(s, tok);
         return hipGetLastError();
     }
+    if (const int depth = p.upb_fwd >= p.units ? team_fwd_depth(p, t, a) : 0) {
+        const int tok = prof_begin(s, silu ? "gn_silu_team_fwd" : "gn_team_fwd");
+        const hipError_t e = launch_team_forward(p, t, a, w.part, depth, s);
+        prof_end(s, tok);
+        return e;
+    }
     const int64_t bpu2 = p.cpg * p.cpp2;  // second-pass blocks per unit
     const char* apply_name = silu ? "gn_silu_apply" : "gn_apply";
     if (fold_ok(p, t, p.upb_fwd)) {
@@ -1784,6 +1790,20 @@ hipError_t launch_backward(const Plan& p, const Tuning& t, const BwdArgs& a, hip
             });
         });
         prof_end(s, tok);
+        return hipGetLastError();
+    }
+    if (p.upb_bwd >= p.units && !recover_lo(a) && team_bwd_fits(p, t, a)) {
+        int tok = prof_begin(s, silu ? "gn_silu_team_bwd" : "gn_team_bwd");
+        const hipError_t e =
+            launch_team_backward(p, t, a, w.part, p.N > 1 ? w.plane_sums : nullptr, s);
+        prof_end(s, tok);
+        if (e != hipSuccess) return e;
+        if (p.N > 1 && (a.dgamma || a.dbeta)) {
+            tok = prof_begin(s, "gn_param_finish");
+            k_param_finish<<<dim3((unsigned)((p.C + 255) / 256)), 256, 0, s>>>(
+                w.plane_sums, a.dgamma, a.dbeta, p.N, p.C);
+            prof_end(s, tok);
+        }
         return hipGetLastError();
     }
     const int64_t bpu2 = p.cpg * p.cpp2;  // second-pass blocks per unit

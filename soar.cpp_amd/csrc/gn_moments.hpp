@@ -34,10 +34,10 @@ __device__ __forceinline__ double2 centred_moments(double S, double Q, double N,
 // square), the wave adds them, and thread 0 re-centres the waves' sums on
 // wave 0's reference in wave order.  lds: 4 * NT / 64 doubles.  Ends with
 // the block synchronised once (the caller synchronises before reusing lds).
-template <int NT>
-__device__ __forceinline__ double2 block_moments(float K, float s_f, float q_f, int cnt,
-                                                 double* lds) {
-    constexpr int W = NT / 64;
+//
+// First the wave: lane 0 writes its (n, S, Q, Rw) to dst[0], dst[step], ...
+__device__ __forceinline__ void wave_moments(float K, float s_f, float q_f, int cnt, double* dst,
+                                             int step) {
     const float Rw = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(K)));
     double S = 0.0, Q = 0.0;
     if (cnt > 0) {
@@ -52,30 +52,40 @@ __device__ __forceinline__ double2 block_moments(float K, float s_f, float q_f, 
     n = wave_sum(n);
     S = wave_sum(S);
     Q = wave_sum(Q);
-    const int t = threadIdx.x, lane = t & 63, w = t >> 6;
-    if (lane == 0) {
-        lds[w] = (double)n;
-        lds[W + w] = S;
-        lds[2 * W + w] = Q;
-        lds[3 * W + w] = (double)Rw;
+    if ((threadIdx.x & 63) == 0) {
+        dst[0] = (double)n;
+        dst[step] = S;
+        dst[2 * step] = Q;
+        dst[3 * step] = (double)Rw;
     }
+}
+
+// Then the W waves' sums (wave i's at src[i], src[step + i], ...), in order.
+template <int W>
+__device__ __forceinline__ double2 combine_wave_moments(const double* src, int step) {
+    const double R0 = src[3 * step];
+    double N = src[0], S0 = src[step], Q0 = src[2 * step];
+#pragma unroll
+    for (int i = 1; i < W; ++i) {
+        const double ni = src[i], Si = src[step + i];
+        if (ni == 0.0) continue;
+        const double d = src[3 * step + i] - R0;
+        const double nd = ni * d;
+        Q0 += fma(d, 2.0 * Si + nd, src[2 * step + i]);
+        S0 += Si + nd;
+        N += ni;
+    }
+    return centred_moments(S0, Q0, N, R0);
+}
+
+template <int NT>
+__device__ __forceinline__ double2 block_moments(float K, float s_f, float q_f, int cnt,
+                                                 double* lds) {
+    constexpr int W = NT / 64;
+    wave_moments(K, s_f, q_f, cnt, lds + (threadIdx.x >> 6), W);
     __syncthreads();
     double2 r = make_double2(0.0, 0.0);
-    if (t == 0) {
-        const double R0 = lds[3 * W];
-        double N = lds[0], S0 = lds[W], Q0 = lds[2 * W];
-#pragma unroll
-        for (int i = 1; i < W; ++i) {
-            const double ni = lds[i], Si = lds[W + i];
-            if (ni == 0.0) continue;
-            const double d = lds[3 * W + i] - R0;
-            const double nd = ni * d;
-            Q0 += fma(d, 2.0 * Si + nd, lds[2 * W + i]);
-            S0 += Si + nd;
-            N += ni;
-        }
-        r = centred_moments(S0, Q0, N, R0);
-    }
+    if (threadIdx.x == 0) r = combine_wave_moments<W>(lds, W);
     return r;
 }
 

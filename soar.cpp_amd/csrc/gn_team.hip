@@ -1,0 +1,758 @@
+// gn_team.hip - GroupNorm(+SiLU) of large tensors with every unit kept on
+// chip between its two passes.
+//
+// The two-launch path reads a unit twice (statistics, then apply; reduction,
+// then dx): 3 tensor passes forward and 5 backward, each at the rate of the
+// memory.  Here a team of blocks owns a unit: every block loads its share
+// once, reduces it to the chunk partials of the two-launch path, publishes
+// them, waits for the team's other partials, finishes the unit's sums itself
+// and writes y (dx) from what it holds: 2 tensor passes forward, 3 backward.
+//
+// What bounds it: memory, in phases.  A team loads, waits and stores, and
+// while it waits only the next team's blocks load; a copy from registers in
+// such phases takes 375-390 us per 2 GiB moved, a streaming copy 332.  So
+// teams are kept small against the chip (several in flight) where the unit
+// allows.  Measured, two launches -> one (forward; backward), us:
+//   32 x 512^2, 8 groups    21 -> 15.5;  34 -> 22
+//   64 x 512^2, 16          37 -> 23.5;  58 -> 42
+//   32 x 1024^2, 8          66 -> 49;    106 -> 85-93
+//   64 x 1024^2, 16         123 -> 99;   203 -> 170-187
+//   2 x 128 x 1024^2, 32    490 -> 380-399; 811 -> 670-756
+//   64 x 2048^2, 16         491 -> 436-450; (too large)
+// Held on chip per block: 512 threads at 128 VGPRs, two blocks per CU, so up
+// to 32 (64) floats of x per thread in registers and 16 more in LDS forward,
+// 32 of x and 32 of dy backward.  (Backward with a further chunk in LDS, for
+// units of 64 MB, gained 4% and needed the whole chip to itself; reading x
+// again instead of holding it was slower than two launches.)
+//
+// Every chunk (8192 floats of a plane, 256 threads of 8 vectors) and output
+// uses the arithmetic of k_stats / k_apply / k_bwd_reduce / k_bwd_dx in the
+// same order.  The finishes add the chunks' partials lane by lane (thread by
+// thread) and then the lanes by a tree; a block takes the chunks of whole
+// lanes ("items") and publishes the lanes' sums, at most a few hundred per
+// unit.  So the sums are the two-launch path's up to the order of their
+// float64 additions.  (The forward's moments are taken about the unit's first
+// value and not about its first partial's mean, which no other block knows.)
+//
+// Hand-off.  A sum is two 64-bit words in a slot that the launch before
+// (k_team_clear) set to all ones, a NaN that no partial is (publish maps it to
+// another).  Words are written and read with relaxed atomics of device scope,
+// which go past the XCDs' private caches; a reader needs no flag and no fence,
+// since it takes a slot's words as they turn valid.
+//
+// Every wait ends.  The blocks of a team are consecutive, so they normally
+// run together; but nothing guarantees it (other work on the device, fewer
+// CUs).  A block that has waited `limit` clock ticks computes the missing
+// sums itself, from memory, with the owner's arithmetic, and publishes them;
+// owner and helper write the same bits.  So no block depends on another one
+// running.  (Which is why outputs that overlap inputs take the two launches.)
+#include <algorithm>
+#include <atomic>
+#include <type_traits>
+
+#include "gn_internal.hpp"
+#include "gn_math.hpp"
+#include "gn_moments.hpp"
+#include "soar_gn.h"
+
+// Lambdas that take a chunk's registers are always inlined: a call would put
+// them in memory.
+#define SOAR_INLINE __attribute__((always_inline))
+
+namespace soar {
+namespace gn {
+namespace {
+
+typedef float f4 __attribute__((ext_vector_type(4)));
+typedef unsigned long long u64;
+
+constexpr int kTeamThreads = 512;
+constexpr int kHalf = 256;     // threads of a half-block, which walks whole chunks
+constexpr int kVec = 8;        // vectors of a chunk per thread
+constexpr int kTeamChunk = 4 * kVec * kHalf;  // 8192 floats
+constexpr int kMaxItems = 1024;                // per unit
+constexpr int kMaxCpg = 128;                  // channels per unit
+// Blocks of a team, of the 512 that 256 CUs hold: with fewer, the team after
+// it is already loading, and work of other streams on some CUs does not keep
+// a team from running together.
+constexpr int kMaxTeam = 400;
+// Chunks of the tensor (32 MB).  Below, both ways live in the caches and the
+// launches decide, of which this way has one more each way and dgamma's with
+// several samples: 2 x 32 x 256^2 with residual, 512 chunks, forward and
+// backward 37.3 us as two launches each, 39.9 here; 32 x 512^2, 1024 chunks,
+// 54.6 and 38.
+constexpr int64_t kTeamMinChunks = 1024;
+constexpr u64 kUnset = ~0ull;
+
+__device__ __forceinline__ u64 load_word(const u64* p) {
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+__device__ __forceinline__ void publish(u64* slot, double a, double b) {
+    u64 wa = __builtin_bit_cast(u64, a), wb = __builtin_bit_cast(u64, b);
+    if (wa == kUnset) wa = 0x7ff8000000000000ull;
+    if (wb == kUnset) wb = 0x7ff8000000000000ull;
+    __hip_atomic_store(slot, wa, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __hip_atomic_store(slot + 1, wb, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+__global__ __launch_bounds__(256) void k_team_clear(u64* __restrict__ slots, int64_t words) {
+    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (i < words) slots[i] = kUnset;
+}
+
+// Geometry of a team launch.  Item `it` of a unit is the chunks that lane
+// r = it % lanes of span it / lanes adds: r, r + lanes, ... of the span's
+// chunks (forward: one span, the unit; backward: a span per plane).
+struct Team {
+    int64_t C, G, HW;
+    int cpg, cpp, P;      // channels per unit, chunks per plane and per unit
+    int span, lanes, nq;  // chunks of a span, its lanes, chunks of a lane (at most)
+    int items, ipb;       // of a unit, of a block
+    int blocks;           // per unit
+    u64 limit;            // clock ticks (100 MHz) a block waits for the others
+};
+
+// Chunk number of item it's i-th chunk, or -1.
+__device__ __forceinline__ int item_chunk(const Team& g, int it, int i) {
+    const int sp = it / g.lanes, c = it - sp * g.lanes + i * g.lanes;
+    return it < g.items && c < g.span ? sp * g.span + c : -1;
+}
+
+// Chunk c of unit u: its plane, first element and length (0 for c < 0).
+struct TeamChunk {
+    int64_t plane, base;
+    int len;
+};
+__device__ __forceinline__ TeamChunk team_chunk(const Team& g, int64_t u, int c) {
+    const int c0 = max(c, 0), pl = c0 / g.cpp, k = c0 - pl * g.cpp;
+    TeamChunk r;
+    r.plane = u * g.cpg + pl;
+    r.base = r.plane * g.HW + (int64_t)k * kTeamChunk;
+    r.len = c < 0 ? 0 : (int)min<int64_t>(kTeamChunk, g.HW - (int64_t)k * kTeamChunk);
+    return r;
+}
+
+// A chunk's vectors, thread t's at t, t + 256, ...: through a raw buffer
+// descriptor of the chunk, so vectors past its end (all of them for a chunk
+// that is not there) load zeros and store nothing, without a branch.
+__device__ __forceinline__ auto chunk_buffer(const float* x, const TeamChunk& c) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(x + c.base), (short)0, 4 * c.len,
+                                             0x00020000);
+}
+constexpr int kNonTemporal = 2;  // cache policy bit of the buffer accesses
+
+__device__ __forceinline__ void load_chunk(f4 (&v)[kVec], const float* __restrict__ x,
+                                           const TeamChunk& c, int t) {
+    const auto rs = chunk_buffer(x, c);
+#pragma unroll
+    for (int k = 0; k < kVec; ++k)
+        v[k] = __builtin_bit_cast(
+            f4, __builtin_amdgcn_raw_buffer_load_b128(rs, 16 * (t + k * kHalf), 0,
+                                                      kNonTemporal));
+}
+
+// One vector (the waits' fallback: few registers beside the held chunks).
+__device__ __forceinline__ f4 load_vec(const float* __restrict__ x, const TeamChunk& c, int i) {
+    return __builtin_bit_cast(
+        f4, __builtin_amdgcn_raw_buffer_load_b128(chunk_buffer(x, c), 16 * i, 0, 0));
+}
+
+__device__ __forceinline__ void store_vec(f4 o, float* __restrict__ y, const TeamChunk& c, int i) {
+    typedef unsigned u4 __attribute__((ext_vector_type(4)));
+    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u4, o), chunk_buffer(y, c), 16 * i, 0,
+                                           kNonTemporal);
+}
+
+// The value of slot `it` once it is set; false when the limit passes first
+// (wave-uniform).  A wait costs one round trip past the caches per look.  (With
+// a slot per chunk, 2048 per 64 MB unit, the looks of 256 blocks were 19 MB
+// each and a unit waited 7 us.  16-byte loads with the scope bits of a
+// volatile buffer load, sc0 sc1, kept returning old words; these are sc1.)
+__device__ __forceinline__ bool poll(double2& v, const u64* __restrict__ slots, int it,
+                                     const Team& g, u64 t0) {
+    const u64* s = slots + 2 * min(it, g.items - 1);
+    for (;;) {
+        const u64 a = load_word(s), b = load_word(s + 1);
+        v = make_double2(__builtin_bit_cast(double, a), __builtin_bit_cast(double, b));
+        if (!__any(a == kUnset || b == kUnset)) return true;
+        if (__builtin_amdgcn_s_memrealtime() - t0 > g.limit) return false;
+        __builtin_amdgcn_s_sleep(2);
+    }
+}
+
+// Which slots are still unset, as bits in miss[kMaxItems / 32].
+__device__ __forceinline__ void team_missing(const u64* __restrict__ slots, const Team& g,
+                                             unsigned* __restrict__ miss) {
+    for (int i = threadIdx.x; i < kMaxItems / 32; i += kTeamThreads) miss[i] = 0;
+    lds_barrier();
+    for (int j = threadIdx.x; j < g.items; j += kTeamThreads)
+        if (load_word(slots + 2 * j) == kUnset || load_word(slots + 2 * j + 1) == kUnset)
+            atomicOr(&miss[j >> 5], 1u << (j & 31));
+    lds_barrier();
+}
+
+// Whether item `it` is still to be computed by this block (block-uniform):
+// unset before and now, so that the waiting blocks, which begin at their own
+// items, share the work.  Two barriers for an item that was missing.
+__device__ __forceinline__ bool team_take(const u64* __restrict__ slots, int it,
+                                          unsigned* __restrict__ miss) {
+    const unsigned bit = 1u << (it & 31);
+    if (!(miss[it >> 5] & bit)) return false;
+    lds_barrier();  // every thread has read the bit
+    if (threadIdx.x == 0 && load_word(slots + 2 * it) != kUnset &&
+        load_word(slots + 2 * it + 1) != kUnset)
+        miss[it >> 5] &= ~bit;
+    lds_barrier();
+    return miss[it >> 5] & bit;
+}
+
+// ---- forward -----------------------------------------------------------------
+
+// k_stats' sums of a chunk, for a thread of 256: shift K, sums, count.  get(k)
+// is the thread's vector k.
+struct ChunkSums {
+    float K, s, q;
+    int cnt;
+};
+template <int UNROLL, typename F>
+__device__ __forceinline__ ChunkSums chunk_sums(F&& get, int len, int t) {
+    ChunkSums r;
+    r.K = get(0).x;
+    const int n4 = len >> 2;
+    r.cnt = t < n4 ? 4 * ((n4 - 1 - t) / kHalf + 1) : 0;
+    float s0 = 0.f, s1 = 0.f, s2 = 0.f, s3 = 0.f, q0 = 0.f, q1 = 0.f, q2 = 0.f, q3 = 0.f;
+    // (a vector past the chunk's end counts as K: it adds zeros)
+    const bool whole = len == kTeamChunk;
+#pragma unroll UNROLL
+    for (int k = 0; k < kVec; ++k) {
+        f4 x = get(k);
+        if (!whole && 4 * k >= r.cnt) x = f4{r.K, r.K, r.K, r.K};
+        const float d0 = x.x - r.K, d1 = x.y - r.K, d2 = x.z - r.K, d3 = x.w - r.K;
+        s0 += d0;
+        s1 += d1;
+        s2 += d2;
+        s3 += d3;
+        q0 = fmaf(d0, d0, q0);
+        q1 = fmaf(d1, d1, q1);
+        q2 = fmaf(d2, d2, q2);
+        q3 = fmaf(d3, d3, q3);
+    }
+    r.s = (s0 + s1) + (s2 + s3);
+    r.q = (q0 + q1) + (q2 + q3);
+    return r;
+}
+
+// NR chunks per half-block in registers (32 VGPRs each), NL in LDS (64 KB
+// for both half-blocks); RES: y += x.
+template <int NR, int NL, bool SILU, bool RES>
+__global__ __launch_bounds__(kTeamThreads, 4) void k_team_fwd(
+    const float* __restrict__ x, const float* __restrict__ gamma, const float* __restrict__ beta,
+    float* __restrict__ y, float* __restrict__ mean, float* __restrict__ rstd,
+    float* __restrict__ mean_lo, u64* __restrict__ all_slots, Team g, float eps) {
+    constexpr int NQ = NR + NL;  // chunks per half-block
+    static_assert(NL <= 1 && NR >= 1, "at most one LDS chunk per half-block");
+    __shared__ f4 hold[NL > 0 ? NL * 2 * kVec * kHalf : 1];
+    __shared__ double mom[2 * NQ][16];  // (n, S, Q, Rw) x 4 waves of each chunk
+    __shared__ double2 cm[2 * NQ];      // and its (mean, M2)
+    __shared__ unsigned miss[kMaxItems / 32];
+    __shared__ double2 sums[kHalf / 64];
+    __shared__ float bc[3];
+    __shared__ int late;
+    const int hb = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 8);  // half-block
+    const int t = threadIdx.x & (kHalf - 1), w = t >> 6;
+    const int64_t u = blockIdx.x / (unsigned)g.blocks;
+    const int kb = (int)(blockIdx.x - (unsigned)u * g.blocks);
+    u64* __restrict__ slots = all_slots + 2 * u * g.items;
+    // chunk m of the block: chunk m % nq of its item m / nq (-1: none)
+    auto block_chunk = [&](int m) {
+        const int o = m / g.nq;
+        return o < g.ipb ? item_chunk(g, kb * g.ipb + o, m - o * g.nq) : -1;
+    };
+    auto chunk_no = [&](int q) { return block_chunk(2 * q + hb); };
+    const double R = (double)x[u * g.cpg * g.HW];  // the moments' reference
+    // an item's sums about R from its chunks' moments, in order (finish_unit)
+    auto add_chunk = [&](double2& s, const double2& m, int c) {
+        const int k = c % g.cpp;
+        const double n = (double)min<int64_t>(kTeamChunk, g.HW - (int64_t)k * kTeamChunk);
+        const double d = m.x - R, nd = n * d;
+        s.x += nd;
+        s.y += fma(nd, d, m.y);
+    };
+    auto sum_chunk = [&](const f4 (&v)[kVec], int q, int len) SOAR_INLINE {
+        const ChunkSums r = chunk_sums<kVec>([&](int k) SOAR_INLINE { return v[k]; }, len, t);
+        wave_moments(r.K, r.s, r.q, r.cnt, &mom[2 * q + hb][w], 4);
+    };
+
+    f4 v[NR][kVec];
+    auto load_q = [&](f4 (&r)[kVec], int q) SOAR_INLINE {
+        load_chunk(r, x, team_chunk(g, u, chunk_no(q)), t);
+    };
+    if constexpr (NL > 0) {
+        // (the last register chunk waits for the LDS chunk's registers)
+        f4 l[kVec];
+        load_q(l, 0);
+#pragma unroll
+        for (int i = 0; i < NR - 1; ++i) load_q(v[i], NL + i);
+        __builtin_amdgcn_sched_barrier(0);
+        sum_chunk(l, 0, team_chunk(g, u, chunk_no(0)).len);
+#pragma unroll
+        for (int k = 0; k < kVec; ++k) hold[(hb * kVec + k) * kHalf + t] = l[k];
+        __builtin_amdgcn_sched_barrier(0);
+        load_q(v[NR - 1], NL + NR - 1);
+    } else {
+#pragma unroll
+        for (int i = 0; i < NR; ++i) load_q(v[i], i);
+    }
+#pragma unroll
+    for (int i = 0; i < NR; ++i)
+        sum_chunk(v[i], NL + i, team_chunk(g, u, chunk_no(NL + i)).len);
+    lds_barrier();
+    if (threadIdx.x < 2 * NQ) cm[threadIdx.x] = combine_wave_moments<4>(mom[threadIdx.x], 4);
+    lds_barrier();
+    if ((int)threadIdx.x < g.ipb && kb * g.ipb + (int)threadIdx.x < g.items) {
+        double2 s = make_double2(0.0, 0.0);
+        for (int i = 0; i < g.nq; ++i) {
+            const int m = threadIdx.x * g.nq + i, c = block_chunk(m);
+            if (c >= 0) add_chunk(s, cm[m], c);
+        }
+        publish(slots + 2 * (kb * g.ipb + threadIdx.x), s.x, s.y);
+    }
+    // the unit's sums over the items, on half-block 0
+    auto gather = [&] {
+        if (threadIdx.x == 0) late = 0;
+        lds_barrier();
+        if (hb == 0) {
+            const u64 t0 = __builtin_amdgcn_s_memrealtime();
+            double2 v = make_double2(0.0, 0.0);
+            for (int it = t; it - t < g.items; it += kHalf) {
+                double2 p;
+                if (!poll(p, slots, it, g, t0)) late = 1;
+                if (it < g.items) {
+                    v.x += p.x;
+                    v.y += p.y;
+                }
+            }
+            v.x = wave_sum(v.x);
+            v.y = wave_sum(v.y);
+            if ((t & 63) == 0) sums[w] = v;
+        }
+        lds_barrier();
+        const bool done = late == 0;
+        lds_barrier();
+        return done;
+    };
+    if (!gather()) {
+        // compute what is missing (block-uniform loops; half-block 0 works)
+        team_missing(slots, g, miss);
+        for (int j = 0, it = kb * g.ipb; j < g.items; ++j, ++it) {
+            if (it >= g.items) it = 0;
+            if (!team_take(slots, it, miss)) continue;
+            double2 s = make_double2(0.0, 0.0);  // thread 0's
+            for (int i = 0; i < g.nq; ++i) {
+                const int c = item_chunk(g, it, i);
+                if (c < 0) continue;
+                if (hb == 0) {
+                    const TeamChunk ck = team_chunk(g, u, c);
+                    const ChunkSums cs = chunk_sums<1>(
+                        [&](int k) SOAR_INLINE { return load_vec(x, ck, t + k * kHalf); }, ck.len, t);
+                    wave_moments(cs.K, cs.s, cs.q, cs.cnt, &mom[0][w], 4);
+                }
+                lds_barrier();
+                if (threadIdx.x == 0) add_chunk(s, combine_wave_moments<4>(mom[0], 4), c);
+                lds_barrier();
+            }
+            if (threadIdx.x == 0) publish(slots + 2 * it, s.x, s.y);
+        }
+        // (every slot is set or its words are on their way)
+        while (!gather()) {}
+    }
+    if (threadIdx.x == 0) {
+        double S = sums[0].x, Q = sums[0].y;
+#pragma unroll
+        for (int i = 1; i < kHalf / 64; ++i) {
+            S += sums[i].x;
+            Q += sums[i].y;
+        }
+        const double n = (double)(g.cpg * g.HW);
+        const double2 mm = centred_moments(S, Q, n, R);
+        const double var = mm.y / n;
+        const float hi = (float)mm.x, lo = (float)(mm.x - (double)hi);
+        const float r = (float)(1.0 / sqrt(var + (double)eps));
+        bc[0] = hi;
+        bc[1] = r;
+        bc[2] = lo;
+        if (kb == 0) {
+            mean[u] = hi;
+            rstd[u] = r;
+            if (mean_lo) mean_lo[u] = lo;
+        }
+    }
+    lds_barrier();
+    const float mu = bc[0], rs = bc[1], e = -bc[2] * rs;
+    // k_apply
+    auto apply = [&](const f4 (&d)[kVec], int c) SOAR_INLINE {
+        const TeamChunk ck = team_chunk(g, u, c);
+        const int64_t ch = ck.plane % g.C;
+        const float gm = gamma ? gamma[ch] : 1.0f;
+        const float a = gm * rs, b = fmaf(gm, e, beta ? beta[ch] : 0.0f);
+#pragma unroll
+        for (int k = 0; k < kVec; ++k) {
+            f4 o;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const float z = fmaf(d[k][i] - mu, a, b);
+                o[i] = SILU ? silu_fast(z) : z;
+                if (RES) o[i] += d[k][i];
+            }
+            store_vec(o, y, ck, t + k * kHalf);
+        }
+    };
+#pragma unroll
+    for (int i = 0; i < NR; ++i) apply(v[i], chunk_no(NL + i));
+    if constexpr (NL > 0) {
+        f4 l[kVec];
+#pragma unroll
+        for (int k = 0; k < kVec; ++k) l[k] = hold[(hb * kVec + k) * kHalf + t];
+        apply(l, chunk_no(0));
+    }
+}
+
+// ---- backward ----------------------------------------------------------------
+
+// k_bwd_reduce's sums of a chunk for a thread of 256; with KEEP the dz
+// replace the dy.  (A vector past the chunk's end has dy = 0 and adds zeros.)
+struct BwdCoef {
+    float mu, r, e, gm, bt;
+};
+template <bool SILU, bool KEEP>
+__device__ __forceinline__ void add_bwd_vec(const f4& x, f4& dy, const BwdCoef& k, float (&sa)[2],
+                                            float (&sb)[2]) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const float xh = fmaf(x[i] - k.mu, k.r, k.e);
+        const float dz = SILU ? dsilu_fast(dy[i], fmaf(k.gm, xh, k.bt)) : dy[i];
+        sa[i & 1] += dz;
+        sb[i & 1] = fmaf(dz, xh, sb[i & 1]);
+        if (KEEP) dy[i] = dz;
+    }
+}
+template <bool SILU, bool KEEP>
+__device__ __forceinline__ float2 chunk_bwd_sums(const f4 (&v)[kVec], f4 (&dy)[kVec],
+                                                 const BwdCoef& k) {
+    float sa[2] = {0.f, 0.f}, sb[2] = {0.f, 0.f};
+#pragma unroll
+    for (int q = 0; q < kVec; ++q) {
+        add_bwd_vec<SILU, KEEP>(v[q], dy[q], k, sa, sb);
+        if (q % 2 == 1)  // (or the vectors' work is interleaved and spills)
+            __builtin_amdgcn_sched_barrier(0);
+    }
+    return make_float2(sa[0] + sa[1], sb[0] + sb[1]);
+}
+
+// One chunk (x and dy) per half-block, in registers.  RES: dx += dy, so dy is
+// kept and dz formed again; else dz takes dy's place.
+template <bool SILU, bool RES>
+__global__ __launch_bounds__(kTeamThreads, 4) void k_team_bwd(
+    const float* __restrict__ dy, const float* __restrict__ x, const float* __restrict__ gamma,
+    const float* __restrict__ beta, const float* __restrict__ mean,
+    const float* __restrict__ rstd, const float* __restrict__ mean_lo, float* __restrict__ dx,
+    float* __restrict__ dgamma, float* __restrict__ dbeta, double2* __restrict__ plane_sums,
+    u64* __restrict__ all_slots, Team g) {
+    constexpr bool KEEP = SILU && !RES;
+    __shared__ float2 wsum[2][4];
+    __shared__ unsigned miss[kMaxItems / 32];
+    __shared__ double2 gsum[kHalf];
+    __shared__ double2 psum[kMaxCpg];  // the unit's plane sums (its first block)
+    __shared__ float bc[2];
+    __shared__ int late;
+    const int hb = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 8);
+    const int t = threadIdx.x & (kHalf - 1), w = t >> 6;
+    const int64_t u = blockIdx.x / (unsigned)g.blocks;
+    const int kb = (int)(blockIdx.x - (unsigned)u * g.blocks);
+    u64* __restrict__ slots = all_slots + 2 * u * g.items;
+    const float mu = mean[u], r = rstd[u], e = mean_lo ? -mean_lo[u] * r : 0.0f;
+    auto block_chunk = [&](int m) {
+        const int o = m / g.nq;
+        return o < g.ipb ? item_chunk(g, kb * g.ipb + o, m - o * g.nq) : -1;
+    };
+    auto coef = [&](const TeamChunk& c) {
+        const int64_t ch = c.plane % g.C;
+        return BwdCoef{mu, r, e, gamma ? gamma[ch] : 1.0f, beta ? beta[ch] : 0.0f};
+    };
+    auto reduce = [&](float2 s, float2* dst) {  // block_sum2's wave part
+        s.x = wave_sum(s.x);
+        s.y = wave_sum(s.y);
+        if ((t & 63) == 0) dst[w] = s;
+    };
+    auto wave_total = [](const float2* s) {  // and its sum over the waves
+        float2 a = s[0];
+#pragma unroll
+        for (int i = 1; i < 4; ++i) {
+            a.x += s[i].x;
+            a.y += s[i].y;
+        }
+        return a;
+    };
+
+    const TeamChunk ck = team_chunk(g, u, block_chunk(hb));
+    const BwdCoef k = coef(ck);
+    f4 v[kVec], d[kVec];
+    load_chunk(v, x, ck, t);
+    load_chunk(d, dy, ck, t);
+    reduce(chunk_bwd_sums<SILU, KEEP>(v, d, k), wsum[hb]);
+    lds_barrier();
+    if ((int)threadIdx.x < g.ipb && kb * g.ipb + (int)threadIdx.x < g.items) {
+        double A = 0.0, B = 0.0;
+        for (int i = 0; i < g.nq; ++i) {
+            const int m = threadIdx.x * g.nq + i;
+            if (block_chunk(m) < 0) continue;
+            const float2 s = wave_total(wsum[m]);
+            A += (double)s.x;
+            B += (double)s.y;
+        }
+        publish(slots + 2 * (kb * g.ipb + threadIdx.x), A, B);
+    }
+    // finish_bwd_unit on half-block 0: groups of gs lanes, a plane each
+    const int gs = bwd_plane_lanes(g.lanes), ngroups = kHalf / gs;
+    auto gather = [&] {
+        if (threadIdx.x == 0) late = 0;
+        lds_barrier();
+        if (hb == 0) {
+            const u64 t0 = __builtin_amdgcn_s_memrealtime();
+            const int grp = t / gs, rr = t & (gs - 1);
+            double S1 = 0.0, S2 = 0.0;
+            for (int j = grp; j - grp < g.cpg; j += ngroups) {
+                const bool mine = j < g.cpg;
+                double A = 0.0, B = 0.0;
+                for (int q = rr; q - rr < g.lanes; q += gs) {
+                    double2 v;
+                    if (!poll(v, slots, j * g.lanes + min(q, g.lanes - 1), g, t0)) late = 1;
+                    if (mine && q < g.lanes) {
+                        A += v.x;
+                        B += v.y;
+                    }
+                }
+                for (int off = gs >> 1; off > 0; off >>= 1) {
+                    A += __shfl_xor(A, off);
+                    B += __shfl_xor(B, off);
+                }
+                if (mine && rr == 0) {
+                    const int64_t ch = (u * g.cpg + j) % g.C;
+                    if (kb == 0) psum[j] = make_double2(A, B);
+                    const double gj = gamma ? (double)gamma[ch] : 1.0;
+                    S1 += gj * A;
+                    S2 += gj * B;
+                }
+            }
+            if (rr == 0) gsum[grp] = make_double2(S1, S2);
+        }
+        lds_barrier();
+        const bool done = late == 0;
+        lds_barrier();
+        return done;
+    };
+    if (!gather()) {
+        // compute what is missing (block-uniform loops; half-block 0 works)
+        team_missing(slots, g, miss);
+        for (int j = 0, it = kb * g.ipb; j < g.items; ++j, ++it) {
+            if (it >= g.items) it = 0;
+            if (!team_take(slots, it, miss)) continue;
+            double A = 0.0, B = 0.0;  // thread 0's
+            for (int i = 0; i < g.nq; ++i) {
+                const int c = item_chunk(g, it, i);
+                if (c < 0) continue;
+                if (hb == 0) {
+                    const TeamChunk cm = team_chunk(g, u, c);
+                    const BwdCoef km = coef(cm);
+                    float sa[2] = {0.f, 0.f}, sb[2] = {0.f, 0.f};
+#pragma unroll 1
+                    for (int q = 0; q < kVec; ++q) {
+                        f4 b = load_vec(dy, cm, t + q * kHalf);
+                        add_bwd_vec<SILU, false>(load_vec(x, cm, t + q * kHalf), b, km, sa, sb);
+                    }
+                    reduce(make_float2(sa[0] + sa[1], sb[0] + sb[1]), wsum[0]);
+                }
+                lds_barrier();
+                if (threadIdx.x == 0) {
+                    const float2 s = wave_total(wsum[0]);
+                    A += (double)s.x;
+                    B += (double)s.y;
+                }
+                lds_barrier();
+            }
+            if (threadIdx.x == 0) publish(slots + 2 * it, A, B);
+        }
+        while (!gather()) {}
+    }
+    if (kb == 0) {
+        for (int j = threadIdx.x; j < g.cpg; j += kTeamThreads) {
+            const int64_t plane = u * g.cpg + j, ch = plane % g.C;
+            const double2 s = psum[j];
+            if (plane_sums) {
+                plane_sums[plane] = s;
+            } else {  // one sample: k_param_finish's sums are these
+                if (dbeta) dbeta[ch] = (float)((double)dbeta[ch] + s.x);
+                if (dgamma) dgamma[ch] = (float)((double)dgamma[ch] + s.y);
+            }
+        }
+    }
+    if (threadIdx.x == 0) {
+        double s1 = 0.0, s2 = 0.0;
+        for (int i = 0; i < ngroups; ++i) {
+            s1 += gsum[i].x;
+            s2 += gsum[i].y;
+        }
+        const double Md = (double)(g.cpg * g.HW);
+        bc[0] = (float)(-(double)r * s1 / Md);
+        bc[1] = (float)(-(double)r * s2 / Md);
+    }
+    lds_barrier();
+    const float B = bc[0], D = bc[1];
+    // k_bwd_dx
+    const float A = k.gm * r;
+#pragma unroll
+    for (int q = 0; q < kVec; ++q) {
+        f4 o;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const float xh = fmaf(v[q][i] - mu, r, e);
+            const float dz = SILU && !KEEP ? dsilu_fast(d[q][i], fmaf(k.gm, xh, k.bt)) : d[q][i];
+            o[i] = fmaf(A, dz, fmaf(D, xh, B));
+            if (RES) o[i] += d[q][i];
+        }
+        store_vec(o, dx, ck, t + q * kHalf);
+        if (q % 2 == 1) __builtin_amdgcn_sched_barrier(0);
+    }
+}
+
+template <typename F>
+void bsel(bool b, F&& f) {
+    if (b)
+        f(std::true_type{});
+    else
+        f(std::false_type{});
+}
+
+// CUs of the current device (a property of the device, asked once each).
+int device_cus() {
+    static std::atomic<int> cus[64];
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 0;
+    int n = cus[dev].load(std::memory_order_relaxed);
+    if (n == 0) {
+        if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
+            return 0;
+        cus[dev].store(n, std::memory_order_relaxed);
+    }
+    return n;
+}
+
+// Geometry for `depth` chunks per half-block: a block is one item of 2 depth
+// chunks, or (backward) several planes of fewer.
+Team team_of(const Plan& p, const Tuning& t, bool bwd, int depth) {
+    Team g;
+    g.C = p.C;
+    g.G = p.G;
+    g.HW = p.HW;
+    g.cpg = (int)p.cpg;
+    g.cpp = (int)p.cpp;
+    g.P = (int)(p.cpg * p.cpp);
+    const int n = 2 * depth;  // chunks of a block
+    g.span = bwd ? g.cpp : g.P;
+    g.nq = std::min(n, g.span);
+    g.lanes = (g.span + g.nq - 1) / g.nq;
+    g.items = g.P / g.span * g.lanes;
+    g.ipb = n / g.nq;
+    g.blocks = (g.items + g.ipb - 1) / g.ipb;
+    g.limit = (u64)t.team_wait_us * 100;
+    return g;
+}
+
+bool team_fits(const Plan& p, const Tuning& t, const Team& g) {
+    return t.team_wait_us >= 0 && p.chunk == kTeamChunk && p.HW % 4 == 0 && p.cpg <= kMaxCpg &&
+           p.cpg * p.cpp <= (int64_t)1 << 20 && p.units * p.cpg * p.cpp < (int64_t)1 << 30 &&
+           g.items <= kMaxItems && g.blocks <= kMaxTeam * device_cus() / 256;
+}
+
+void launch_clear(const Plan& p, const Team& g, double2* slots, hipStream_t s) {
+    const int64_t words = 2 * p.units * g.items;
+    k_team_clear<<<dim3((unsigned)((words + 255) / 256)), 256, 0, s>>>(reinterpret_cast<u64*>(slots),
+                                                                      words);
+}
+
+bool aligned(const void* p) { return ((uintptr_t)p & 15) == 0; }
+
+// Outputs written over inputs stay with the two launches: a block that
+// computes another's sums reads inputs while others already write.
+bool overlap(const Plan& p, const float* a, const float* b) {
+    const int64_t n = p.planes * p.HW;
+    return (uintptr_t)a < (uintptr_t)(b + n) && (uintptr_t)b < (uintptr_t)(a + n);
+}
+
+}  // namespace
+
+// Chunks per half-block, 0: two launches.  One if the tensor's blocks are at
+// most two waves of the chip (64 x 512^2, 2048 chunks: 23.6 us at two chunks,
+// 26.0 at one), else two: half the slots to look at.  Three (LDS) only for
+// units that need it (64 x 2048^2: 448 us; with 512 blocks of two, 436, but
+// such a team needs the whole chip).
+int team_fwd_depth(const Plan& p, const Tuning& t, const FwdArgs& a) {
+    const int64_t chunks = p.units * p.cpg * p.cpp;
+    if (a.res || !aligned(a.x) || !aligned(a.y) || overlap(p, a.x, a.y)) return 0;
+    if (chunks < kTeamMinChunks) return 0;
+    for (int depth = chunks <= 4 * device_cus() ? 1 : 2; depth <= 3; ++depth)
+        if (team_fits(p, t, team_of(p, t, false, depth))) return depth;
+    return 0;
+}
+
+// Units of at most 800 chunks (26 MB) backward: the size of a team.
+bool team_bwd_fits(const Plan& p, const Tuning& t, const BwdArgs& a) {
+    return a.dx && !(a.flags & SOAR_GN_ACCUMULATE_DX) && aligned(a.x) && aligned(a.dy) &&
+           aligned(a.dx) && !overlap(p, a.x, a.dx) && !overlap(p, a.dy, a.dx) &&
+           p.units * p.cpg * p.cpp >= kTeamMinChunks &&
+           team_fits(p, t, team_of(p, t, true, 1));
+}
+
+hipError_t launch_team_forward(const Plan& p, const Tuning& t, const FwdArgs& a, double2* part,
+                               int depth, hipStream_t s) {
+    const Team g = team_of(p, t, false, depth);
+    launch_clear(p, g, part, s);
+    const dim3 grid((unsigned)(p.units * g.blocks));
+    bsel((a.flags & SOAR_GN_SILU) != 0, [&](auto S) {
+        bsel((a.flags & SOAR_GN_RESIDUAL) != 0, [&](auto R) {
+            auto go = [&](auto NR, auto NL) {
+                k_team_fwd<NR(), NL(), S(), R()><<<grid, kTeamThreads, 0, s>>>(
+                    a.x, a.gamma, a.beta, a.y, a.mean, a.rstd, a.mean_lo,
+                    reinterpret_cast<u64*>(part), g, a.eps);
+            };
+            using Z = std::integral_constant<int, 0>;
+            using I1 = std::integral_constant<int, 1>;
+            using I2 = std::integral_constant<int, 2>;
+            switch (depth) {
+                case 1: go(I1{}, Z{}); break;
+                case 2: go(I2{}, Z{}); break;
+                default: go(I2{}, I1{});
+            }
+        });
+    });
+    return hipGetLastError();
+}
+
+hipError_t launch_team_backward(const Plan& p, const Tuning& t, const BwdArgs& a, double2* part,
+                                double2* plane_sums, hipStream_t s) {
+    const Team g = team_of(p, t, true, 1);
+    launch_clear(p, g, part, s);
+    const dim3 grid((unsigned)(p.units * g.blocks));
+    bsel((a.flags & SOAR_GN_SILU) != 0, [&](auto S) {
+        bsel((a.flags & SOAR_GN_RESIDUAL) != 0, [&](auto R) {
+            k_team_bwd<S(), R()><<<grid, kTeamThreads, 0, s>>>(
+                a.dy, a.x, a.gamma, a.beta, a.mean, a.rstd, a.mean_lo, a.dx, a.dgamma, a.dbeta,
+                plane_sums, reinterpret_cast<u64*>(part), g);
+        });
+    });
+    return hipGetLastError();
+}
+
+}  // namespace gn
+}  // namespace soar

@@ -60,6 +60,7 @@ TUNE_PW_CBA_MIN = 16
 TUNE_PW_CBA_BLOCKS = 17
 TUNE_DW_CBA_MIN = 18
 TUNE_NT_TAIL_MB = 19
+TUNE_TEAM_WAIT_US = 20
 
 
 class SoarUnavailable(RuntimeError):
