@@ -206,6 +206,11 @@ SOAR_API int soar_add_backward(const float* grad_y, float* grad_a,
 SOAR_API int soar_zero(float* ptr, size_t n, void* stream);
 SOAR_API int soar_fill(float* ptr, float value, size_t n, void* stream);
 
+/* soar_zero of up to three buffers in one launch (fresh gradients before an
+ * accumulating backward); a length of 0 skips its buffer. */
+SOAR_API int soar_zero3(float* a, size_t na, float* b, size_t nb, float* c,
+                        size_t nc, void* stream);
+
 /* ---- pointwise convolution, the producer of CBA's GroupNorm ---------- */
 /* The 1x1 / stride 1 / no-padding / groups 1 convolution of CBA blocks
  * (Down.pw, LKR.pw1/pw2, Ctx.cv1/cv2; src/nn/blocks.cpp:429-480) is a GEMM

@@ -1319,6 +1319,19 @@ SOAR_API int soar_fill(float* ptr, float value, size_t n, void* stream) {
 
 SOAR_API int soar_zero(float* ptr, size_t n, void* stream) { return soar_fill(ptr, 0.0f, n, stream); }
 
+SOAR_API int soar_zero3(float* a, size_t na, float* b, size_t nb, float* c, size_t nc,
+                        void* stream) {
+    if ((na | nb | nc) > (size_t)1 << 60) return fail(SOAR_EINVAL, "too many elements");
+    SOAR_ELEMWISE_PRELUDE(na + nb + nc);
+    int rc;
+    if ((na && (rc = check_dev(a, na * 4, "a"))) || (nb && (rc = check_dev(b, nb * 4, "b"))) ||
+        (nc && (rc = check_dev(c, nc * 4, "c"))))
+        return rc;
+    hipError_t e = soar::gn::launch_zero3(a, (int64_t)na, b, (int64_t)nb, c, (int64_t)nc,
+                                          static_cast<hipStream_t>(stream));
+    return e == hipSuccess ? ok() : hip_fail(e, "zero launch");
+}
+
 // ---- arena -------------------------------------------------------------------
 
 struct soar_arena {

@@ -192,6 +192,29 @@ hipError_t launch_add_backward(const float* gy, float* ga, float* gb, int64_t n,
     return hipGetLastError();
 }
 
+// Fresh gradient buffers: a layer's two or three are a few KB each, so the
+// launch decides; one for all of them.
+__global__ __launch_bounds__(256) void k_zero3(float* __restrict__ a, int64_t na,
+                                               float* __restrict__ b, int64_t nb,
+                                               float* __restrict__ c, int64_t nc) {
+    const int64_t stride = (int64_t)gridDim.x * blockDim.x;
+    for (int64_t j = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; j < na + nb + nc;
+         j += stride) {
+        if (j < na)
+            a[j] = 0.0f;
+        else if (j < na + nb)
+            b[j - na] = 0.0f;
+        else
+            c[j - na - nb] = 0.0f;
+    }
+}
+
+hipError_t launch_zero3(float* a, int64_t na, float* b, int64_t nb, float* c, int64_t nc,
+                        hipStream_t s) {
+    k_zero3<<<grid_for(na + nb + nc), 256, 0, s>>>(a, na, b, nb, c, nc);
+    return hipGetLastError();
+}
+
 hipError_t launch_fill(float* p, float v, int64_t n, hipStream_t s) {
     int tok = prof_begin(s, "fill");
     if (aligned16(p))

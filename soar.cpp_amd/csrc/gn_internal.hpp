@@ -447,6 +447,8 @@ hipError_t launch_add_forward(const float* a, const float* b, float* y,
 hipError_t launch_add_backward(const float* gy, float* ga, float* gb,
                                int64_t n, hipStream_t s);
 hipError_t launch_fill(float* p, float v, int64_t n, hipStream_t s);
+hipError_t launch_zero3(float* a, int64_t na, float* b, int64_t nb, float* c, int64_t nc,
+                        hipStream_t s);
 
 // Deferred weight-gradient finishes (wfinish.hip).  An entry adds
 // sum_g part[g][e] (float64, k_sum_partials' order) into out0[e] (kk1 = 0)

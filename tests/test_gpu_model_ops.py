@@ -658,3 +658,15 @@ def test_fused_clip_adamw_tail(env, max_norm, zero):
     assert L.soar_adamw_clip_multi_tensor_device(None, None, None, None, None, 0, None, 0.9,
                                                  0.999, 1e-8, 0.0, None, 0, 1.0, None, 2,
                                                  None) == gn.SOAR_EINVAL
+
+
+@pytest.mark.parametrize("sizes", [(1, 0, 0), (0, 3, 0), (300, 1, 257), (0, 0, 0), (5, 70000, 64)])
+def test_zero3_clears_each_buffer_and_nothing_else(gpu, sizes):
+    import torch
+    bufs = [torch.full((n + 8,), 3.0, device="cuda") for n in sizes]
+    args = [v for b, n in zip(bufs, sizes) for v in (b[4:].data_ptr() if n else None, n)]
+    gpu.check(gpu.lib().soar_zero3(*args, torch.cuda.current_stream().cuda_stream))
+    for b, n in zip(bufs, sizes):
+        assert not b[4:4 + n].any() and (b[:4] == 3).all() and (b[4 + n:] == 3).all()
+    with pytest.raises(gpu.SoarError):
+        gpu.check(gpu.lib().soar_zero3(None, 4, None, 0, None, 0, None))
