@@ -76,12 +76,13 @@ constexpr int kMaxCpg = 128;                  // channels per unit
 // it is already loading, and work of other streams on some CUs does not keep
 // a team from running together.
 constexpr int kMaxTeam = 400;
-// Chunks of the tensor (32 MB).  Below, both ways live in the caches and the
+// Chunks of the tensor (24 MB).  Below, both ways live in the caches and the
 // launches decide, of which this way has one more each way and dgamma's with
-// several samples: 2 x 32 x 256^2 with residual, 512 chunks, forward and
-// backward 37.3 us as two launches each, 39.9 here; 32 x 512^2, 1024 chunks,
-// 54.6 and 38.
-constexpr int64_t kTeamMinChunks = 1024;
+// several samples.  Forward; backward, us, two launches -> one: 256 chunks
+// 9.3 -> 10.1; 12.1 -> 12.8, 512 (64 x 256^2) 11.4 -> 11.4; 19.5 -> 14.9 (but
+// 20.4 -> 21.3 with residual and two samples), 768 (96 x 256^2) 17.0 -> 13.2;
+// 26.5 -> 20.2, 1024 (32 x 512^2) 21.1 -> 15.8; 33.1 -> 22.3.
+constexpr int64_t kTeamMinChunks = 768;
 constexpr u64 kUnset = ~0ull;
 
 __device__ __forceinline__ u64 load_word(const u64* p) {

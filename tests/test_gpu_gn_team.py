@@ -12,8 +12,8 @@ pytestmark = pytest.mark.gpu
 
 CASES = [
     # (N, C, HW, G, silu, residual, affine)
-    (1, 1024, 8192, 8, True, False, True),       # one chunk per plane, 1024 in all: the least
-    (2, 256, 8196, 4, True, True, True),         # a last chunk of one vector
+    (1, 768, 8192, 8, True, False, True),        # one chunk per plane, 768 in all: the least
+    (2, 192, 8196, 4, True, True, True),         # a last chunk of one vector
     (3, 96, 25600, 8, False, False, True),       # plain GroupNorm, a ragged last chunk
     (1, 32, 262144, 32, True, False, False),     # one plane per unit, no affine
     (2, 64, 65536, 8, False, True, True),
