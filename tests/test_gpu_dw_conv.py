@@ -215,3 +215,37 @@ def test_dw_paths_are_deterministic(gpu, K, S, D, H):
         runs.append([t.cpu().numpy() for t in (y, dx, dw, db)])
     for a, c in zip(*runs):
         assert np.array_equal(a, c)
+
+
+@pytest.mark.parametrize("shape", [(1, 4, 70, 130, 3, 1, 1), (2, 3, 67, 131, 3, 2, 1),
+                                   (1, 3, 45, 203, 7, 1, 1), (1, 2, 50, 66, 5, 1, 1)])
+@pytest.mark.parametrize("accumulate", [False, True])
+def test_rows_at_any_alignment(gpu, shape, accumulate):
+    """Tensors one float past a 16-byte boundary: the same values as aligned
+    ones, and nothing written beside them."""
+    import torch
+    N, C, H, W, K, s, d = shape
+    pad = autopad(K, d)
+    x, w, b = (dev(v) for v in inputs(5, N, C, H, W, K))
+
+    def off(t):
+        buf = torch.full((t.numel() + 8,), 7.0, device="cuda")
+        buf[1:1 + t.numel()] = t.reshape(-1)
+        return buf, buf[1:1 + t.numel()].view(t.shape)
+
+    x = x.view(N, C, H, W)
+    w = w.view(C, K, K)
+    y = gpu.dw_conv_forward(x, w, b, pad, s, d)
+    dy = torch.randn_like(y)
+    dx0 = torch.randn_like(x)
+    want = gpu.dw_conv_backward(dy, x, w, pad, s, d, dx=dx0.clone(), accumulate_dx=accumulate)
+    ybuf, yo = off(torch.zeros_like(y))
+    gpu.dw_conv_forward(off(x)[1], w, b, pad, s, d, y=yo)
+    dbuf, dxo = off(dx0)
+    got = gpu.dw_conv_backward(off(dy)[1], off(x)[1], w, pad, s, d, dx=dxo,
+                               accumulate_dx=accumulate)
+    assert torch.equal(yo, y)
+    for a, t in zip(got, want):
+        assert torch.equal(a, t)
+    for buf in (ybuf, dbuf):
+        assert buf[0] == 7 and (buf[-7:] == 7).all()
