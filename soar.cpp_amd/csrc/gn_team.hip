@@ -12,13 +12,14 @@
 // while it waits only the next team's blocks load; a copy from registers in
 // such phases takes 375-390 us per 2 GiB moved, a streaming copy 332.  So
 // teams are kept small against the chip (several in flight) where the unit
-// allows.  Measured, two launches -> one (forward; backward), us:
-//   32 x 512^2, 8 groups    21 -> 15.5;  34 -> 22
-//   64 x 512^2, 16          37 -> 23.5;  58 -> 42
-//   32 x 1024^2, 8          66 -> 49;    106 -> 85-93
-//   64 x 1024^2, 16         123 -> 99;   203 -> 170-187
-//   2 x 128 x 1024^2, 32    490 -> 380-399; 811 -> 670-756
-//   64 x 2048^2, 16         491 -> 436-450; (too large)
+// allows.  Measured with SiLU, two launches -> one (forward; backward; backward
+// without SiLU), us:
+//   32 x 512^2, 8 groups    21.6 -> 16.5; 33.6 -> 23.1; 32.1 -> 21.7
+//   64 x 512^2, 16          36.8 -> 26.0; 59.2 -> 43.8; 57.4 -> 39.9
+//   32 x 1024^2, 8          66.1 -> 51.3; 104 -> 94;    103 -> 85
+//   64 x 1024^2, 16         125 -> 101;   204 -> 189;   203 -> 168
+//   2 x 128 x 1024^2, 32    490 -> 401;   815 -> 761;   817 -> 667
+//   64 x 2048^2, 16         491 -> 436-458; (too large)
 // Held on chip per block: 512 threads at 128 VGPRs, two blocks per CU, so up
 // to 32 (64) floats of x per thread in registers and 16 more in LDS forward,
 // 32 of x and 32 of dy backward.  (Backward with a further chunk in LDS, for
@@ -83,6 +84,12 @@ constexpr int kMaxTeam = 400;
 // 20.4 -> 21.3 with residual and two samples), 768 (96 x 256^2) 17.0 -> 13.2;
 // 26.5 -> 20.2, 1024 (32 x 512^2) 21.1 -> 15.8; 33.1 -> 22.3.
 constexpr int64_t kTeamMinChunks = 768;
+// Chunks up to which a backward with residual and SiLU comes here (64 MB): its
+// dy stays held and the SiLU's derivative is formed again after the wait.  Two
+// launches -> one, us: 32 x 512^2 32.8 -> 26.0, 64 x 512^2 60.2 -> 50.0, 32 x
+// 1024^2 104.0 -> 102.6, 64 x 1024^2 203 -> 206, 2 x 128 x 1024^2 812 -> 830.
+// (gamma r dz + dy in dy's place instead: 73 spilled registers, 1199.)
+constexpr int64_t kTeamMaxResChunks = 2048;
 constexpr u64 kUnset = ~0ull;
 
 __device__ __forceinline__ u64 load_word(const u64* p) {
@@ -709,9 +716,11 @@ int team_fwd_depth(const Plan& p, const Tuning& t, const FwdArgs& a) {
 
 // Units of at most 800 chunks (26 MB) backward: the size of a team.
 bool team_bwd_fits(const Plan& p, const Tuning& t, const BwdArgs& a) {
+    const bool res_silu = (a.flags & SOAR_GN_RESIDUAL) && (a.flags & SOAR_GN_SILU);
     return a.dx && !(a.flags & SOAR_GN_ACCUMULATE_DX) && aligned(a.x) && aligned(a.dy) &&
            aligned(a.dx) && !overlap(p, a.x, a.dx) && !overlap(p, a.dy, a.dx) &&
            p.units * p.cpg * p.cpp >= kTeamMinChunks &&
+           !(res_silu && p.units * p.cpg * p.cpp > kTeamMaxResChunks) &&
            team_fits(p, t, team_of(p, t, true, 1));
 }
 
