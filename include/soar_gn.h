@@ -609,8 +609,10 @@ SOAR_API int soar_prof_summary(char* buf, size_t buflen);
 #define SOAR_TUNE_TEAM_WAIT_US 20 /* GroupNorm of large units in one pass: */
                                 /* microseconds a block waits for the    */
                                 /* sums of its unit's other blocks       */
-                                /* before it computes the missing ones   */
-                                /* (-1 = two passes instead)             */
+                                /* before it leaves its share to the     */
+                                /* launch after (-1 = two passes         */
+                                /* instead; -2 = every block leaves: for */
+                                /* tests)                                */
 SOAR_API int soar_gn_tune(int key, int64_t value);
 SOAR_API int64_t soar_gn_tune_get(int key);
 

@@ -1605,8 +1605,8 @@ SOAR_API int soar_gn_tune(int key, int64_t value) {
             g_tune.nt_tail_mb = value;
             return ok();
         case SOAR_TUNE_TEAM_WAIT_US:
-            if (value < -1 || value > 1000000)
-                return fail(SOAR_EINVAL, "team_wait_us must be in [-1, 10^6]");
+            if (value < soar::gn::kTeamLeave || value > 1000000)
+                return fail(SOAR_EINVAL, "team_wait_us must be in [-2, 10^6]");
             g_tune.team_wait_us = value;
             return ok();
         default:

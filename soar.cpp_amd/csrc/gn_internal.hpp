@@ -103,9 +103,8 @@ struct Tuning {
                                  // from which the fused kernel runs (0:
                                  // never)
     int64_t team_wait_us = 200;  // gn_team.hip: microseconds a block waits for
-                                 // its team's partials before it computes the
-                                 // missing ones itself (negative: that path
-                                 // is not taken)
+                                 // its team's sums before it leaves its share
+                                 // to the launch after; or kTeamOff, kTeamLeave
     int64_t pw_cba_blocks = 256;  // and the blocks its pixel chunks aim for
                                   // (one per CU: at 64 -> 64 channels over
                                   // 2048^2 pixels 1.03 ms, 1.13 at 512,
@@ -176,15 +175,27 @@ hipError_t launch_forward(const Plan& p, const Tuning& t, const FwdArgs& a,
 hipError_t launch_backward(const Plan& p, const Tuning& t, const BwdArgs& a,
                            hipStream_t s);
 
+// Values of team_wait_us besides a time: the path is not taken; every block
+// leaves (the waits' end, for tests).
+constexpr int64_t kTeamOff = -1, kTeamLeave = -2;
+
+// That path's parts of the workspace: slots of the blocks' sums (the chunk
+// partials' region), a mark that some block left (the unit sums') and the
+// units' marks (the low means').
+struct TeamWs {
+    unsigned long long* slots = nullptr;
+    unsigned long long* any = nullptr;
+    unsigned* left = nullptr;
+};
+
 // Units kept on chip between the passes (gn_team.hip): whether the forward
-// (its depth, 0: not) and the backward of a plan take that path; `part` is the
-// workspace's chunk-partial region.  The backward adds dgamma / dbeta itself,
+// (its depth, 0: not) and the backward of a plan take that path.  The backward adds dgamma / dbeta itself,
 // or with plane_sums (several samples) leaves every plane's sums there.
 int team_fwd_depth(const Plan& p, const Tuning& t, const FwdArgs& a);
 bool team_bwd_fits(const Plan& p, const Tuning& t, const BwdArgs& a);
-hipError_t launch_team_forward(const Plan& p, const Tuning& t, const FwdArgs& a, double2* part,
+hipError_t launch_team_forward(const Plan& p, const Tuning& t, const FwdArgs& a, const TeamWs& w,
                                int depth, hipStream_t s);
-hipError_t launch_team_backward(const Plan& p, const Tuning& t, const BwdArgs& a, double2* part,
+hipError_t launch_team_backward(const Plan& p, const Tuning& t, const BwdArgs& a, const TeamWs& w,
                                 double2* plane_sums, hipStream_t s);
 
 // True when the backward of this plan runs the one-launch small-unit kernel.

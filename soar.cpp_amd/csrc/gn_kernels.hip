@@ -1297,6 +1297,12 @@ WsView ws_view(const Plan& p, void* ws) {
     return v;
 }
 
+TeamWs team_ws(const WsView& v) {
+    typedef unsigned long long u64;
+    return TeamWs{reinterpret_cast<u64*>(v.part), reinterpret_cast<u64*>(v.unit_sums),
+                  reinterpret_cast<unsigned*>(v.lo)};
+}
+
 // Calls f(std::integral_constant<int, U>) for U = 8 or 4 loads in flight.
 template <typename F>
 void loads_sel(int loads, F&& f) {
@@ -1632,7 +1638,7 @@ hipError_t launch_forward(const Plan& p, const Tuning& t, const FwdArgs& a, hipS
     }
     if (const int depth = p.upb_fwd >= p.units ? team_fwd_depth(p, t, a) : 0) {
         const int tok = prof_begin(s, silu ? "gn_silu_team_fwd" : "gn_team_fwd");
-        const hipError_t e = launch_team_forward(p, t, a, w.part, depth, s);
+        const hipError_t e = launch_team_forward(p, t, a, team_ws(w), depth, s);
         prof_end(s, tok);
         return e;
     }
@@ -1795,7 +1801,7 @@ hipError_t launch_backward(const Plan& p, const Tuning& t, const BwdArgs& a, hip
     if (p.upb_bwd >= p.units && !recover_lo(a) && team_bwd_fits(p, t, a)) {
         int tok = prof_begin(s, silu ? "gn_silu_team_bwd" : "gn_team_bwd");
         const hipError_t e =
-            launch_team_backward(p, t, a, w.part, p.N > 1 ? w.plane_sums : nullptr, s);
+            launch_team_backward(p, t, a, team_ws(w), p.N > 1 ? w.plane_sums : nullptr, s);
         prof_end(s, tok);
         if (e != hipSuccess) return e;
         if (p.N > 1 && (a.dgamma || a.dbeta)) {

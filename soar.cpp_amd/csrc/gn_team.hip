@@ -42,11 +42,17 @@
 // since it takes a slot's words as they turn valid.
 //
 // Every wait ends.  The blocks of a team are consecutive, so they normally
-// run together; but nothing guarantees it (other work on the device, fewer
-// CUs).  A block that has waited `limit` clock ticks computes the missing
-// sums itself, from memory, with the owner's arithmetic, and publishes them;
-// owner and helper write the same bits.  So no block depends on another one
-// running.  (Which is why outputs that overlap inputs take the two launches.)
+// run together; but nothing guarantees it (kernels of other streams, fewer
+// CUs).  A block that has waited `limit` clock ticks leaves its share
+// unwritten, with a mark on the unit.  It has published its own sums, so the
+// launch after (k_team_fwd_rest / k_team_bwd_rest) finds all sums of a marked
+// unit in the slots, reads the unit again and writes it, the second pass of
+// two launches; the bits are the same.  No loop ends by another block's
+// store, and once a block of the call has left, the others do not wait
+// either, so a call that meets other work costs one limit more than two
+// launches.  (A marked unit is read after blocks of it wrote theirs, which
+// is why outputs that overlap inputs take the two launches.)  Where nothing
+// is marked the launch ends at once.
 #include <algorithm>
 #include <atomic>
 #include <type_traits>
@@ -104,9 +110,21 @@ __device__ __forceinline__ void publish(u64* slot, double a, double b) {
     __hip_atomic_store(slot + 1, wb, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-__global__ __launch_bounds__(256) void k_team_clear(u64* __restrict__ slots, int64_t words) {
+__global__ __launch_bounds__(256) void k_team_clear(TeamWs w, int64_t words, int64_t units) {
     const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (i < words) slots[i] = kUnset;
+    if (i < words) w.slots[i] = kUnset;
+    if (i < units) w.left[i] = 0;  // (a unit has at least two words)
+    if (i == 0) *w.any = 0;
+}
+
+// Marks of a unit's blocks that left: some block, its first block.
+constexpr unsigned kLeft = 1, kLeftFirst = 2;
+
+// A block leaves (thread 0).
+__device__ __forceinline__ void team_leave(const TeamWs& w, int64_t u, int kb) {
+    __hip_atomic_fetch_or(w.left + u, kb == 0 ? kLeft | kLeftFirst : kLeft, __ATOMIC_RELAXED,
+                          __HIP_MEMORY_SCOPE_AGENT);
+    __hip_atomic_store(w.any, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 // Geometry of a team launch.  Item `it` of a unit is the chunks that lane
@@ -119,6 +137,7 @@ struct Team {
     int items, ipb;       // of a unit, of a block
     int blocks;           // per unit
     u64 limit;            // clock ticks (100 MHz) a block waits for the others
+    int leave;            // every block leaves
 };
 
 // Chunk number of item it's i-th chunk, or -1.
@@ -160,81 +179,59 @@ __device__ __forceinline__ void load_chunk(f4 (&v)[kVec], const float* __restric
                                                       kNonTemporal));
 }
 
-// One vector (the waits' fallback: few registers beside the held chunks).
-__device__ __forceinline__ f4 load_vec(const float* __restrict__ x, const TeamChunk& c, int i) {
-    return __builtin_bit_cast(
-        f4, __builtin_amdgcn_raw_buffer_load_b128(chunk_buffer(x, c), 16 * i, 0, 0));
-}
-
 __device__ __forceinline__ void store_vec(f4 o, float* __restrict__ y, const TeamChunk& c, int i) {
     typedef unsigned u4 __attribute__((ext_vector_type(4)));
     __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u4, o), chunk_buffer(y, c), 16 * i, 0,
                                            kNonTemporal);
 }
 
-// The value of slot `it` once it is set; false when the limit passes first
-// (wave-uniform).  A wait costs one round trip past the caches per look.  (With
+// The value of slot `it` once it is set; false when the limit passes first or
+// another block of the call has left (wave-uniform).  A wait costs one round trip past the caches per look.  (With
 // a slot per chunk, 2048 per 64 MB unit, the looks of 256 blocks were 19 MB
 // each and a unit waited 7 us.  16-byte loads with the scope bits of a
 // volatile buffer load, sc0 sc1, kept returning old words; these are sc1.)
 __device__ __forceinline__ bool poll(double2& v, const u64* __restrict__ slots, int it,
-                                     const Team& g, u64 t0) {
+                                     const Team& g, const TeamWs& w, u64 t0) {
     const u64* s = slots + 2 * min(it, g.items - 1);
     for (;;) {
         const u64 a = load_word(s), b = load_word(s + 1);
         v = make_double2(__builtin_bit_cast(double, a), __builtin_bit_cast(double, b));
         if (!__any(a == kUnset || b == kUnset)) return true;
-        if (__builtin_amdgcn_s_memrealtime() - t0 > g.limit) return false;
+        const bool others = __builtin_amdgcn_readfirstlane((int)load_word(w.any)) != 0;
+        if (others || __builtin_amdgcn_s_memrealtime() - t0 > g.limit) return false;
         __builtin_amdgcn_s_sleep(2);
     }
 }
-
-// Which slots are still unset, as bits in miss[kMaxItems / 32].
-__device__ __forceinline__ void team_missing(const u64* __restrict__ slots, const Team& g,
-                                             unsigned* __restrict__ miss) {
-    for (int i = threadIdx.x; i < kMaxItems / 32; i += kTeamThreads) miss[i] = 0;
-    lds_barrier();
-    for (int j = threadIdx.x; j < g.items; j += kTeamThreads)
-        if (load_word(slots + 2 * j) == kUnset || load_word(slots + 2 * j + 1) == kUnset)
-            atomicOr(&miss[j >> 5], 1u << (j & 31));
-    lds_barrier();
+// The same after the launch that set it.
+__device__ __forceinline__ double2 read_slot(const u64* __restrict__ slots, int it, const Team& g) {
+    const u64* s = slots + 2 * min(it, g.items - 1);
+    return make_double2(__builtin_bit_cast(double, s[0]), __builtin_bit_cast(double, s[1]));
 }
 
-// Whether item `it` is still to be computed by this block (block-uniform):
-// unset before and now, so that the waiting blocks, which begin at their own
-// items, share the work.  Two barriers for an item that was missing.
-__device__ __forceinline__ bool team_take(const u64* __restrict__ slots, int it,
-                                          unsigned* __restrict__ miss) {
-    const unsigned bit = 1u << (it & 31);
-    if (!(miss[it >> 5] & bit)) return false;
-    lds_barrier();  // every thread has read the bit
-    if (threadIdx.x == 0 && load_word(slots + 2 * it) != kUnset &&
-        load_word(slots + 2 * it + 1) != kUnset)
-        miss[it >> 5] &= ~bit;
-    lds_barrier();
-    return miss[it >> 5] & bit;
+// Chunk m of block kb: chunk m % nq of its item m / nq (-1: none).
+__device__ __forceinline__ int block_chunk(const Team& g, int kb, int m) {
+    const int o = m / g.nq;
+    return o < g.ipb ? item_chunk(g, kb * g.ipb + o, m - o * g.nq) : -1;
 }
 
 // ---- forward -----------------------------------------------------------------
 
-// k_stats' sums of a chunk, for a thread of 256: shift K, sums, count.  get(k)
-// is the thread's vector k.
+// k_stats' sums of a chunk, for a thread of 256: shift K, sums, count.
 struct ChunkSums {
     float K, s, q;
     int cnt;
 };
-template <int UNROLL, typename F>
-__device__ __forceinline__ ChunkSums chunk_sums(F&& get, int len, int t) {
+__device__ __forceinline__ ChunkSums chunk_sums(const f4 (&v)[kVec], int len, int t) {
     ChunkSums r;
-    r.K = get(0).x;
+    r.K = v[0].x;
     const int n4 = len >> 2;
     r.cnt = t < n4 ? 4 * ((n4 - 1 - t) / kHalf + 1) : 0;
     float s0 = 0.f, s1 = 0.f, s2 = 0.f, s3 = 0.f, q0 = 0.f, q1 = 0.f, q2 = 0.f, q3 = 0.f;
     // (a vector past the chunk's end counts as K: it adds zeros)
     const bool whole = len == kTeamChunk;
-#pragma unroll UNROLL
+#pragma unroll
     for (int k = 0; k < kVec; ++k) {
-        f4 x = get(k);
+        f4 x = v[k];
         if (!whole && 4 * k >= r.cnt) x = f4{r.K, r.K, r.K, r.K};
         const float d0 = x.x - r.K, d1 = x.y - r.K, d2 = x.z - r.K, d3 = x.w - r.K;
         s0 += d0;
@@ -251,19 +248,86 @@ __device__ __forceinline__ ChunkSums chunk_sums(F&& get, int len, int t) {
     return r;
 }
 
+// The unit's sums over its items, by half-block 0 (thread t of it) into sums:
+// get(it, p): item it's sums, false if they are not there.
+template <typename F>
+__device__ __forceinline__ void gather_fwd(const Team& g, int t, double2* sums, int* late, F get) {
+    double2 v = make_double2(0.0, 0.0);
+    for (int it = t; it - t < g.items; it += kHalf) {
+        double2 p;
+        if (!get(it, p)) *late = 1;
+        if (it < g.items) {
+            v.x += p.x;
+            v.y += p.y;
+        }
+    }
+    v.x = wave_sum(v.x);
+    v.y = wave_sum(v.y);
+    if ((t & 63) == 0) sums[t >> 6] = v;
+}
+
+// Mean, rstd and the mean's low part from them, into bc (thread 0); R: the
+// moments' reference.
+__device__ __forceinline__ void finish_fwd(const Team& g, const double2* sums, double R, float eps,
+                                           int64_t u, bool first, float* __restrict__ mean,
+                                           float* __restrict__ rstd, float* __restrict__ mean_lo,
+                                           float* bc) {
+    double S = sums[0].x, Q = sums[0].y;
+#pragma unroll
+    for (int i = 1; i < kHalf / 64; ++i) {
+        S += sums[i].x;
+        Q += sums[i].y;
+    }
+    const double n = (double)(g.cpg * g.HW);
+    const double2 mm = centred_moments(S, Q, n, R);
+    const double var = mm.y / n;
+    const float hi = (float)mm.x, lo = (float)(mm.x - (double)hi);
+    const float r = (float)(1.0 / sqrt(var + (double)eps));
+    bc[0] = hi;
+    bc[1] = r;
+    bc[2] = lo;
+    if (first) {
+        mean[u] = hi;
+        rstd[u] = r;
+        if (mean_lo) mean_lo[u] = lo;
+    }
+}
+
+// k_apply of a chunk that is held.
+template <bool SILU, bool RES>
+__device__ __forceinline__ void apply_chunk(const f4 (&d)[kVec], const Team& g, const TeamChunk& ck,
+                                            const float* __restrict__ gamma,
+                                            const float* __restrict__ beta, const float* bc,
+                                            float* __restrict__ y, int t) {
+    const float mu = bc[0], rs = bc[1], e = -bc[2] * rs;
+    const int64_t ch = ck.plane % g.C;
+    const float gm = gamma ? gamma[ch] : 1.0f;
+    const float a = gm * rs, b = fmaf(gm, e, beta ? beta[ch] : 0.0f);
+#pragma unroll
+    for (int k = 0; k < kVec; ++k) {
+        f4 o;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const float z = fmaf(d[k][i] - mu, a, b);
+            o[i] = SILU ? silu_fast(z) : z;
+            if (RES) o[i] += d[k][i];
+        }
+        store_vec(o, y, ck, t + k * kHalf);
+    }
+}
+
 // NR chunks per half-block in registers (32 VGPRs each), NL in LDS (64 KB
 // for both half-blocks); RES: y += x.
 template <int NR, int NL, bool SILU, bool RES>
 __global__ __launch_bounds__(kTeamThreads, 4) void k_team_fwd(
     const float* __restrict__ x, const float* __restrict__ gamma, const float* __restrict__ beta,
     float* __restrict__ y, float* __restrict__ mean, float* __restrict__ rstd,
-    float* __restrict__ mean_lo, u64* __restrict__ all_slots, Team g, float eps) {
+    float* __restrict__ mean_lo, TeamWs ws, Team g, float eps) {
     constexpr int NQ = NR + NL;  // chunks per half-block
     static_assert(NL <= 1 && NR >= 1, "at most one LDS chunk per half-block");
     __shared__ f4 hold[NL > 0 ? NL * 2 * kVec * kHalf : 1];
     __shared__ double mom[2 * NQ][16];  // (n, S, Q, Rw) x 4 waves of each chunk
     __shared__ double2 cm[2 * NQ];      // and its (mean, M2)
-    __shared__ unsigned miss[kMaxItems / 32];
     __shared__ double2 sums[kHalf / 64];
     __shared__ float bc[3];
     __shared__ int late;
@@ -271,13 +335,8 @@ __global__ __launch_bounds__(kTeamThreads, 4) void k_team_fwd(
     const int t = threadIdx.x & (kHalf - 1), w = t >> 6;
     const int64_t u = blockIdx.x / (unsigned)g.blocks;
     const int kb = (int)(blockIdx.x - (unsigned)u * g.blocks);
-    u64* __restrict__ slots = all_slots + 2 * u * g.items;
-    // chunk m of the block: chunk m % nq of its item m / nq (-1: none)
-    auto block_chunk = [&](int m) {
-        const int o = m / g.nq;
-        return o < g.ipb ? item_chunk(g, kb * g.ipb + o, m - o * g.nq) : -1;
-    };
-    auto chunk_no = [&](int q) { return block_chunk(2 * q + hb); };
+    u64* __restrict__ slots = ws.slots + 2 * u * g.items;
+    auto chunk_no = [&](int q) { return block_chunk(g, kb, 2 * q + hb); };
     const double R = (double)x[u * g.cpg * g.HW];  // the moments' reference
     // an item's sums about R from its chunks' moments, in order (finish_unit)
     auto add_chunk = [&](double2& s, const double2& m, int c) {
@@ -288,7 +347,7 @@ __global__ __launch_bounds__(kTeamThreads, 4) void k_team_fwd(
         s.y += fma(nd, d, m.y);
     };
     auto sum_chunk = [&](const f4 (&v)[kVec], int q, int len) SOAR_INLINE {
-        const ChunkSums r = chunk_sums<kVec>([&](int k) SOAR_INLINE { return v[k]; }, len, t);
+        const ChunkSums r = chunk_sums(v, len, t);
         wave_moments(r.K, r.s, r.q, r.cnt, &mom[2 * q + hb][w], 4);
     };
 
@@ -321,100 +380,27 @@ __global__ __launch_bounds__(kTeamThreads, 4) void k_team_fwd(
     if ((int)threadIdx.x < g.ipb && kb * g.ipb + (int)threadIdx.x < g.items) {
         double2 s = make_double2(0.0, 0.0);
         for (int i = 0; i < g.nq; ++i) {
-            const int m = threadIdx.x * g.nq + i, c = block_chunk(m);
+            const int m = threadIdx.x * g.nq + i, c = block_chunk(g, kb, m);
             if (c >= 0) add_chunk(s, cm[m], c);
         }
         publish(slots + 2 * (kb * g.ipb + threadIdx.x), s.x, s.y);
     }
-    // the unit's sums over the items, on half-block 0
-    auto gather = [&] {
-        if (threadIdx.x == 0) late = 0;
-        lds_barrier();
-        if (hb == 0) {
-            const u64 t0 = __builtin_amdgcn_s_memrealtime();
-            double2 v = make_double2(0.0, 0.0);
-            for (int it = t; it - t < g.items; it += kHalf) {
-                double2 p;
-                if (!poll(p, slots, it, g, t0)) late = 1;
-                if (it < g.items) {
-                    v.x += p.x;
-                    v.y += p.y;
-                }
-            }
-            v.x = wave_sum(v.x);
-            v.y = wave_sum(v.y);
-            if ((t & 63) == 0) sums[w] = v;
-        }
-        lds_barrier();
-        const bool done = late == 0;
-        lds_barrier();
-        return done;
-    };
-    if (!gather()) {
-        // compute what is missing (block-uniform loops; half-block 0 works)
-        team_missing(slots, g, miss);
-        for (int j = 0, it = kb * g.ipb; j < g.items; ++j, ++it) {
-            if (it >= g.items) it = 0;
-            if (!team_take(slots, it, miss)) continue;
-            double2 s = make_double2(0.0, 0.0);  // thread 0's
-            for (int i = 0; i < g.nq; ++i) {
-                const int c = item_chunk(g, it, i);
-                if (c < 0) continue;
-                if (hb == 0) {
-                    const TeamChunk ck = team_chunk(g, u, c);
-                    const ChunkSums cs = chunk_sums<1>(
-                        [&](int k) SOAR_INLINE { return load_vec(x, ck, t + k * kHalf); }, ck.len, t);
-                    wave_moments(cs.K, cs.s, cs.q, cs.cnt, &mom[0][w], 4);
-                }
-                lds_barrier();
-                if (threadIdx.x == 0) add_chunk(s, combine_wave_moments<4>(mom[0], 4), c);
-                lds_barrier();
-            }
-            if (threadIdx.x == 0) publish(slots + 2 * it, s.x, s.y);
-        }
-        // (every slot is set or its words are on their way)
-        while (!gather()) {}
-    }
-    if (threadIdx.x == 0) {
-        double S = sums[0].x, Q = sums[0].y;
-#pragma unroll
-        for (int i = 1; i < kHalf / 64; ++i) {
-            S += sums[i].x;
-            Q += sums[i].y;
-        }
-        const double n = (double)(g.cpg * g.HW);
-        const double2 mm = centred_moments(S, Q, n, R);
-        const double var = mm.y / n;
-        const float hi = (float)mm.x, lo = (float)(mm.x - (double)hi);
-        const float r = (float)(1.0 / sqrt(var + (double)eps));
-        bc[0] = hi;
-        bc[1] = r;
-        bc[2] = lo;
-        if (kb == 0) {
-            mean[u] = hi;
-            rstd[u] = r;
-            if (mean_lo) mean_lo[u] = lo;
-        }
+    if (threadIdx.x == 0) late = g.leave;
+    lds_barrier();
+    if (hb == 0 && !g.leave) {
+        const u64 t0 = __builtin_amdgcn_s_memrealtime();
+        gather_fwd(g, t, sums, &late,
+                   [&](int it, double2& p) { return poll(p, slots, it, g, ws, t0); });
     }
     lds_barrier();
-    const float mu = bc[0], rs = bc[1], e = -bc[2] * rs;
-    // k_apply
+    if (late) {
+        if (threadIdx.x == 0) team_leave(ws, u, kb);
+        return;  // whole block
+    }
+    if (threadIdx.x == 0) finish_fwd(g, sums, R, eps, u, kb == 0, mean, rstd, mean_lo, bc);
+    lds_barrier();
     auto apply = [&](const f4 (&d)[kVec], int c) SOAR_INLINE {
-        const TeamChunk ck = team_chunk(g, u, c);
-        const int64_t ch = ck.plane % g.C;
-        const float gm = gamma ? gamma[ch] : 1.0f;
-        const float a = gm * rs, b = fmaf(gm, e, beta ? beta[ch] : 0.0f);
-#pragma unroll
-        for (int k = 0; k < kVec; ++k) {
-            f4 o;
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const float z = fmaf(d[k][i] - mu, a, b);
-                o[i] = SILU ? silu_fast(z) : z;
-                if (RES) o[i] += d[k][i];
-            }
-            store_vec(o, y, ck, t + k * kHalf);
-        }
+        apply_chunk<SILU, RES>(d, g, team_chunk(g, u, c), gamma, beta, bc, y, t);
     };
 #pragma unroll
     for (int i = 0; i < NR; ++i) apply(v[i], chunk_no(NL + i));
@@ -423,6 +409,43 @@ __global__ __launch_bounds__(kTeamThreads, 4) void k_team_fwd(
 #pragma unroll
         for (int k = 0; k < kVec; ++k) l[k] = hold[(hb * kVec + k) * kHalf + t];
         apply(l, chunk_no(0));
+    }
+}
+
+// The units that blocks left: `blocks` as k_team_fwd's, 2 depth chunks each.
+template <bool SILU, bool RES>
+__global__ __launch_bounds__(kTeamThreads) void k_team_fwd_rest(
+    const float* __restrict__ x, const float* __restrict__ gamma, const float* __restrict__ beta,
+    float* __restrict__ y, float* __restrict__ mean, float* __restrict__ rstd,
+    float* __restrict__ mean_lo, TeamWs ws, Team g, float eps, int64_t blocks, int depth) {
+    __shared__ double2 sums[kHalf / 64];
+    __shared__ float bc[3];
+    if (*ws.any == 0) return;
+    const int hb = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 8);
+    const int t = threadIdx.x & (kHalf - 1);
+    for (int64_t b = blockIdx.x; b < blocks; b += gridDim.x) {
+        const int64_t u = b / g.blocks;
+        const int kb = (int)(b - u * g.blocks);
+        if (ws.left[u] == 0) continue;
+        const u64* __restrict__ slots = ws.slots + 2 * u * g.items;
+        int late;
+        if (hb == 0)
+            gather_fwd(g, t, sums, &late, [&](int it, double2& p) {
+                p = read_slot(slots, it, g);
+                return true;
+            });
+        lds_barrier();
+        if (threadIdx.x == 0)
+            finish_fwd(g, sums, (double)x[u * g.cpg * g.HW], eps, u, kb == 0, mean, rstd, mean_lo,
+                       bc);
+        lds_barrier();
+        for (int q = 0; q < depth; ++q) {
+            const TeamChunk ck = team_chunk(g, u, block_chunk(g, kb, 2 * q + hb));
+            f4 v[kVec];
+            load_chunk(v, x, ck, t);
+            apply_chunk<SILU, RES>(v, g, ck, gamma, beta, bc, y, t);
+        }
+        lds_barrier();  // sums and bc are free
     }
 }
 
@@ -458,6 +481,106 @@ __device__ __forceinline__ float2 chunk_bwd_sums(const f4 (&v)[kVec], f4 (&dy)[k
     return make_float2(sa[0] + sa[1], sb[0] + sb[1]);
 }
 
+// finish_bwd_unit's sums by half-block 0 (thread t of it): groups of lanes, a
+// plane each, into gsum, and the planes' own into psum (when `planes`).
+// get(it, v) as in gather_fwd.
+template <typename F>
+__device__ __forceinline__ void gather_bwd(const Team& g, int t, int64_t u, bool planes,
+                                           const float* __restrict__ gamma, double2* gsum,
+                                           double2* psum, int* late, F get) {
+    const int gs = bwd_plane_lanes(g.lanes), ngroups = kHalf / gs;
+    const int grp = t / gs, rr = t & (gs - 1);
+    double S1 = 0.0, S2 = 0.0;
+    for (int j = grp; j - grp < g.cpg; j += ngroups) {
+        const bool mine = j < g.cpg;
+        double A = 0.0, B = 0.0;
+        for (int q = rr; q - rr < g.lanes; q += gs) {
+            double2 v;
+            if (!get(j * g.lanes + min(q, g.lanes - 1), v)) *late = 1;
+            if (mine && q < g.lanes) {
+                A += v.x;
+                B += v.y;
+            }
+        }
+        for (int off = gs >> 1; off > 0; off >>= 1) {
+            A += __shfl_xor(A, off);
+            B += __shfl_xor(B, off);
+        }
+        if (mine && rr == 0) {
+            const int64_t ch = (u * g.cpg + j) % g.C;
+            if (planes) psum[j] = make_double2(A, B);
+            const double gj = gamma ? (double)gamma[ch] : 1.0;
+            S1 += gj * A;
+            S2 += gj * B;
+        }
+    }
+    if (rr == 0) gsum[grp] = make_double2(S1, S2);
+}
+
+// The planes' sums (the unit's first block): to plane_sums, or, with one
+// sample, k_param_finish's additions.
+__device__ __forceinline__ void give_planes(const Team& g, int64_t u, const double2* psum,
+                                            double2* __restrict__ plane_sums,
+                                            float* __restrict__ dgamma, float* __restrict__ dbeta) {
+    for (int j = threadIdx.x; j < g.cpg; j += kTeamThreads) {
+        const int64_t plane = u * g.cpg + j, ch = plane % g.C;
+        const double2 s = psum[j];
+        if (plane_sums) {
+            plane_sums[plane] = s;
+        } else {
+            if (dbeta) dbeta[ch] = (float)((double)dbeta[ch] + s.x);
+            if (dgamma) dgamma[ch] = (float)((double)dgamma[ch] + s.y);
+        }
+    }
+}
+
+// dx's two unit coefficients, into bc (thread 0).
+__device__ __forceinline__ void finish_bwd(const Team& g, const double2* gsum, float r, float* bc) {
+    const int ngroups = kHalf / bwd_plane_lanes(g.lanes);
+    double s1 = 0.0, s2 = 0.0;
+    for (int i = 0; i < ngroups; ++i) {
+        s1 += gsum[i].x;
+        s2 += gsum[i].y;
+    }
+    const double Md = (double)(g.cpg * g.HW);
+    bc[0] = (float)(-(double)r * s1 / Md);
+    bc[1] = (float)(-(double)r * s2 / Md);
+}
+
+// k_bwd_dx of a chunk that is held; DZ: d holds dz.
+template <bool SILU, bool RES, bool DZ>
+__device__ __forceinline__ void dx_chunk(const f4 (&v)[kVec], const f4 (&d)[kVec],
+                                         const TeamChunk& ck, const BwdCoef& k, const float* bc,
+                                         float* __restrict__ dx, int t) {
+    const float B = bc[0], D = bc[1];
+    const float A = k.gm * k.r;
+#pragma unroll
+    for (int q = 0; q < kVec; ++q) {
+        f4 o;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const float xh = fmaf(v[q][i] - k.mu, k.r, k.e);
+            const float dz = SILU && !DZ ? dsilu_fast(d[q][i], fmaf(k.gm, xh, k.bt)) : d[q][i];
+            o[i] = fmaf(A, dz, fmaf(D, xh, B));
+            if (RES) o[i] += d[q][i];
+        }
+        store_vec(o, dx, ck, t + q * kHalf);
+        if (q % 2 == 1) __builtin_amdgcn_sched_barrier(0);
+    }
+}
+
+__device__ __forceinline__ BwdCoef bwd_coef(const Team& g, int64_t u, const TeamChunk& c,
+                                            const float* __restrict__ gamma,
+                                            const float* __restrict__ beta,
+                                            const float* __restrict__ mean,
+                                            const float* __restrict__ rstd,
+                                            const float* __restrict__ mean_lo) {
+    const int64_t ch = c.plane % g.C;
+    const float r = rstd[u];
+    return BwdCoef{mean[u], r, mean_lo ? -mean_lo[u] * r : 0.0f, gamma ? gamma[ch] : 1.0f,
+                   beta ? beta[ch] : 0.0f};
+}
+
 // One chunk (x and dy) per half-block, in registers.  RES: dx += dy, so dy is
 // kept and dz formed again; else dz takes dy's place.
 template <bool SILU, bool RES>
@@ -466,10 +589,9 @@ __global__ __launch_bounds__(kTeamThreads, 4) void k_team_bwd(
     const float* __restrict__ beta, const float* __restrict__ mean,
     const float* __restrict__ rstd, const float* __restrict__ mean_lo, float* __restrict__ dx,
     float* __restrict__ dgamma, float* __restrict__ dbeta, double2* __restrict__ plane_sums,
-    u64* __restrict__ all_slots, Team g) {
+    TeamWs ws, Team g) {
     constexpr bool KEEP = SILU && !RES;
     __shared__ float2 wsum[2][4];
-    __shared__ unsigned miss[kMaxItems / 32];
     __shared__ double2 gsum[kHalf];
     __shared__ double2 psum[kMaxCpg];  // the unit's plane sums (its first block)
     __shared__ float bc[2];
@@ -478,16 +600,7 @@ __global__ __launch_bounds__(kTeamThreads, 4) void k_team_bwd(
     const int t = threadIdx.x & (kHalf - 1), w = t >> 6;
     const int64_t u = blockIdx.x / (unsigned)g.blocks;
     const int kb = (int)(blockIdx.x - (unsigned)u * g.blocks);
-    u64* __restrict__ slots = all_slots + 2 * u * g.items;
-    const float mu = mean[u], r = rstd[u], e = mean_lo ? -mean_lo[u] * r : 0.0f;
-    auto block_chunk = [&](int m) {
-        const int o = m / g.nq;
-        return o < g.ipb ? item_chunk(g, kb * g.ipb + o, m - o * g.nq) : -1;
-    };
-    auto coef = [&](const TeamChunk& c) {
-        const int64_t ch = c.plane % g.C;
-        return BwdCoef{mu, r, e, gamma ? gamma[ch] : 1.0f, beta ? beta[ch] : 0.0f};
-    };
+    u64* __restrict__ slots = ws.slots + 2 * u * g.items;
     auto reduce = [&](float2 s, float2* dst) {  // block_sum2's wave part
         s.x = wave_sum(s.x);
         s.y = wave_sum(s.y);
@@ -503,8 +616,8 @@ __global__ __launch_bounds__(kTeamThreads, 4) void k_team_bwd(
         return a;
     };
 
-    const TeamChunk ck = team_chunk(g, u, block_chunk(hb));
-    const BwdCoef k = coef(ck);
+    const TeamChunk ck = team_chunk(g, u, block_chunk(g, kb, hb));
+    const BwdCoef k = bwd_coef(g, u, ck, gamma, beta, mean, rstd, mean_lo);
     f4 v[kVec], d[kVec];
     load_chunk(v, x, ck, t);
     load_chunk(d, dy, ck, t);
@@ -514,123 +627,69 @@ __global__ __launch_bounds__(kTeamThreads, 4) void k_team_bwd(
         double A = 0.0, B = 0.0;
         for (int i = 0; i < g.nq; ++i) {
             const int m = threadIdx.x * g.nq + i;
-            if (block_chunk(m) < 0) continue;
+            if (block_chunk(g, kb, m) < 0) continue;
             const float2 s = wave_total(wsum[m]);
             A += (double)s.x;
             B += (double)s.y;
         }
         publish(slots + 2 * (kb * g.ipb + threadIdx.x), A, B);
     }
-    // finish_bwd_unit on half-block 0: groups of gs lanes, a plane each
-    const int gs = bwd_plane_lanes(g.lanes), ngroups = kHalf / gs;
-    auto gather = [&] {
-        if (threadIdx.x == 0) late = 0;
-        lds_barrier();
-        if (hb == 0) {
-            const u64 t0 = __builtin_amdgcn_s_memrealtime();
-            const int grp = t / gs, rr = t & (gs - 1);
-            double S1 = 0.0, S2 = 0.0;
-            for (int j = grp; j - grp < g.cpg; j += ngroups) {
-                const bool mine = j < g.cpg;
-                double A = 0.0, B = 0.0;
-                for (int q = rr; q - rr < g.lanes; q += gs) {
-                    double2 v;
-                    if (!poll(v, slots, j * g.lanes + min(q, g.lanes - 1), g, t0)) late = 1;
-                    if (mine && q < g.lanes) {
-                        A += v.x;
-                        B += v.y;
-                    }
-                }
-                for (int off = gs >> 1; off > 0; off >>= 1) {
-                    A += __shfl_xor(A, off);
-                    B += __shfl_xor(B, off);
-                }
-                if (mine && rr == 0) {
-                    const int64_t ch = (u * g.cpg + j) % g.C;
-                    if (kb == 0) psum[j] = make_double2(A, B);
-                    const double gj = gamma ? (double)gamma[ch] : 1.0;
-                    S1 += gj * A;
-                    S2 += gj * B;
-                }
-            }
-            if (rr == 0) gsum[grp] = make_double2(S1, S2);
-        }
-        lds_barrier();
-        const bool done = late == 0;
-        lds_barrier();
-        return done;
-    };
-    if (!gather()) {
-        // compute what is missing (block-uniform loops; half-block 0 works)
-        team_missing(slots, g, miss);
-        for (int j = 0, it = kb * g.ipb; j < g.items; ++j, ++it) {
-            if (it >= g.items) it = 0;
-            if (!team_take(slots, it, miss)) continue;
-            double A = 0.0, B = 0.0;  // thread 0's
-            for (int i = 0; i < g.nq; ++i) {
-                const int c = item_chunk(g, it, i);
-                if (c < 0) continue;
-                if (hb == 0) {
-                    const TeamChunk cm = team_chunk(g, u, c);
-                    const BwdCoef km = coef(cm);
-                    float sa[2] = {0.f, 0.f}, sb[2] = {0.f, 0.f};
-#pragma unroll 1
-                    for (int q = 0; q < kVec; ++q) {
-                        f4 b = load_vec(dy, cm, t + q * kHalf);
-                        add_bwd_vec<SILU, false>(load_vec(x, cm, t + q * kHalf), b, km, sa, sb);
-                    }
-                    reduce(make_float2(sa[0] + sa[1], sb[0] + sb[1]), wsum[0]);
-                }
-                lds_barrier();
-                if (threadIdx.x == 0) {
-                    const float2 s = wave_total(wsum[0]);
-                    A += (double)s.x;
-                    B += (double)s.y;
-                }
-                lds_barrier();
-            }
-            if (threadIdx.x == 0) publish(slots + 2 * it, A, B);
-        }
-        while (!gather()) {}
-    }
-    if (kb == 0) {
-        for (int j = threadIdx.x; j < g.cpg; j += kTeamThreads) {
-            const int64_t plane = u * g.cpg + j, ch = plane % g.C;
-            const double2 s = psum[j];
-            if (plane_sums) {
-                plane_sums[plane] = s;
-            } else {  // one sample: k_param_finish's sums are these
-                if (dbeta) dbeta[ch] = (float)((double)dbeta[ch] + s.x);
-                if (dgamma) dgamma[ch] = (float)((double)dgamma[ch] + s.y);
-            }
-        }
-    }
-    if (threadIdx.x == 0) {
-        double s1 = 0.0, s2 = 0.0;
-        for (int i = 0; i < ngroups; ++i) {
-            s1 += gsum[i].x;
-            s2 += gsum[i].y;
-        }
-        const double Md = (double)(g.cpg * g.HW);
-        bc[0] = (float)(-(double)r * s1 / Md);
-        bc[1] = (float)(-(double)r * s2 / Md);
+    if (threadIdx.x == 0) late = g.leave;
+    lds_barrier();
+    if (hb == 0 && !g.leave) {
+        const u64 t0 = __builtin_amdgcn_s_memrealtime();
+        gather_bwd(g, t, u, kb == 0, gamma, gsum, psum, &late,
+                   [&](int it, double2& v) { return poll(v, slots, it, g, ws, t0); });
     }
     lds_barrier();
-    const float B = bc[0], D = bc[1];
-    // k_bwd_dx
-    const float A = k.gm * r;
-#pragma unroll
-    for (int q = 0; q < kVec; ++q) {
-        f4 o;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const float xh = fmaf(v[q][i] - mu, r, e);
-            const float dz = SILU && !KEEP ? dsilu_fast(d[q][i], fmaf(k.gm, xh, k.bt)) : d[q][i];
-            o[i] = fmaf(A, dz, fmaf(D, xh, B));
-            if (RES) o[i] += d[q][i];
-        }
-        store_vec(o, dx, ck, t + q * kHalf);
-        if (q % 2 == 1) __builtin_amdgcn_sched_barrier(0);
+    if (late) {
+        if (threadIdx.x == 0) team_leave(ws, u, kb);
+        return;  // whole block
+    }
+    if (kb == 0) give_planes(g, u, psum, plane_sums, dgamma, dbeta);
+    if (threadIdx.x == 0) finish_bwd(g, gsum, k.r, bc);
+    lds_barrier();
+    dx_chunk<SILU, RES, KEEP>(v, d, ck, k, bc, dx, t);
+}
+
+// The units that blocks left.
+template <bool SILU, bool RES>
+__global__ __launch_bounds__(kTeamThreads) void k_team_bwd_rest(
+    const float* __restrict__ dy, const float* __restrict__ x, const float* __restrict__ gamma,
+    const float* __restrict__ beta, const float* __restrict__ mean,
+    const float* __restrict__ rstd, const float* __restrict__ mean_lo, float* __restrict__ dx,
+    float* __restrict__ dgamma, float* __restrict__ dbeta, double2* __restrict__ plane_sums,
+    TeamWs ws, Team g, int64_t blocks) {
+    __shared__ double2 gsum[kHalf];
+    __shared__ double2 psum[kMaxCpg];
+    __shared__ float bc[2];
+    if (*ws.any == 0) return;
+    const int hb = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 8);
+    const int t = threadIdx.x & (kHalf - 1);
+    for (int64_t b = blockIdx.x; b < blocks; b += gridDim.x) {
+        const int64_t u = b / g.blocks;
+        const int kb = (int)(b - u * g.blocks);
+        const unsigned left = ws.left[u];
+        if (left == 0) continue;
+        const u64* __restrict__ slots = ws.slots + 2 * u * g.items;
+        const TeamChunk ck = team_chunk(g, u, block_chunk(g, kb, hb));
+        const BwdCoef k = bwd_coef(g, u, ck, gamma, beta, mean, rstd, mean_lo);
+        f4 v[kVec], d[kVec];
+        load_chunk(v, x, ck, t);
+        load_chunk(d, dy, ck, t);
+        int late;
+        if (hb == 0)
+            gather_bwd(g, t, u, kb == 0, gamma, gsum, psum, &late, [&](int it, double2& p) {
+                p = read_slot(slots, it, g);
+                return true;
+            });
+        lds_barrier();
+        // (once: a first block that did not leave has added its sums)
+        if (kb == 0 && (left & kLeftFirst)) give_planes(g, u, psum, plane_sums, dgamma, dbeta);
+        if (threadIdx.x == 0) finish_bwd(g, gsum, k.r, bc);
+        lds_barrier();
+        dx_chunk<SILU, RES, false>(v, d, ck, k, bc, dx, t);
+        lds_barrier();  // the shared sums are free
     }
 }
 
@@ -673,26 +732,31 @@ Team team_of(const Plan& p, const Tuning& t, bool bwd, int depth) {
     g.items = g.P / g.span * g.lanes;
     g.ipb = n / g.nq;
     g.blocks = (g.items + g.ipb - 1) / g.ipb;
-    g.limit = (u64)t.team_wait_us * 100;
+    g.limit = (u64)std::max<int64_t>(t.team_wait_us, 0) * 100;
+    g.leave = t.team_wait_us == kTeamLeave;
     return g;
 }
 
 bool team_fits(const Plan& p, const Tuning& t, const Team& g) {
-    return t.team_wait_us >= 0 && p.chunk == kTeamChunk && p.HW % 4 == 0 && p.cpg <= kMaxCpg &&
+    return t.team_wait_us != kTeamOff && p.chunk == kTeamChunk && p.HW % 4 == 0 && p.cpg <= kMaxCpg &&
            p.cpg * p.cpp <= (int64_t)1 << 20 && p.units * p.cpg * p.cpp < (int64_t)1 << 30 &&
            g.items <= kMaxItems && g.blocks <= kMaxTeam * device_cus() / 256;
 }
 
-void launch_clear(const Plan& p, const Team& g, double2* slots, hipStream_t s) {
+void launch_clear(const Plan& p, const Team& g, const TeamWs& w, hipStream_t s) {
     const int64_t words = 2 * p.units * g.items;
-    k_team_clear<<<dim3((unsigned)((words + 255) / 256)), 256, 0, s>>>(reinterpret_cast<u64*>(slots),
-                                                                      words);
+    k_team_clear<<<dim3((unsigned)((words + 255) / 256)), 256, 0, s>>>(w, words, p.units);
+}
+
+// Blocks of the launch for what was left (a block walks several there).
+dim3 rest_grid(int64_t blocks) {
+    return dim3((unsigned)std::min<int64_t>(blocks, 2 * device_cus()));
 }
 
 bool aligned(const void* p) { return ((uintptr_t)p & 15) == 0; }
 
-// Outputs written over inputs stay with the two launches: a block that
-// computes another's sums reads inputs while others already write.
+// Outputs written over inputs stay with the two launches: the launch for what
+// was left reads inputs of blocks that have written.
 bool overlap(const Plan& p, const float* a, const float* b) {
     const int64_t n = p.planes * p.HW;
     return (uintptr_t)a < (uintptr_t)(b + n) && (uintptr_t)b < (uintptr_t)(a + n);
@@ -724,17 +788,17 @@ bool team_bwd_fits(const Plan& p, const Tuning& t, const BwdArgs& a) {
            team_fits(p, t, team_of(p, t, true, 1));
 }
 
-hipError_t launch_team_forward(const Plan& p, const Tuning& t, const FwdArgs& a, double2* part,
+hipError_t launch_team_forward(const Plan& p, const Tuning& t, const FwdArgs& a, const TeamWs& w,
                                int depth, hipStream_t s) {
     const Team g = team_of(p, t, false, depth);
-    launch_clear(p, g, part, s);
-    const dim3 grid((unsigned)(p.units * g.blocks));
+    launch_clear(p, g, w, s);
+    const int64_t blocks = p.units * g.blocks;
+    const dim3 grid((unsigned)blocks);
     bsel((a.flags & SOAR_GN_SILU) != 0, [&](auto S) {
         bsel((a.flags & SOAR_GN_RESIDUAL) != 0, [&](auto R) {
             auto go = [&](auto NR, auto NL) {
                 k_team_fwd<NR(), NL(), S(), R()><<<grid, kTeamThreads, 0, s>>>(
-                    a.x, a.gamma, a.beta, a.y, a.mean, a.rstd, a.mean_lo,
-                    reinterpret_cast<u64*>(part), g, a.eps);
+                    a.x, a.gamma, a.beta, a.y, a.mean, a.rstd, a.mean_lo, w, g, a.eps);
             };
             using Z = std::integral_constant<int, 0>;
             using I1 = std::integral_constant<int, 1>;
@@ -744,21 +808,27 @@ hipError_t launch_team_forward(const Plan& p, const Tuning& t, const FwdArgs& a,
                 case 2: go(I2{}, Z{}); break;
                 default: go(I2{}, I1{});
             }
+            k_team_fwd_rest<S(), R()><<<rest_grid(blocks), kTeamThreads, 0, s>>>(
+                a.x, a.gamma, a.beta, a.y, a.mean, a.rstd, a.mean_lo, w, g, a.eps, blocks, depth);
         });
     });
     return hipGetLastError();
 }
 
-hipError_t launch_team_backward(const Plan& p, const Tuning& t, const BwdArgs& a, double2* part,
+hipError_t launch_team_backward(const Plan& p, const Tuning& t, const BwdArgs& a, const TeamWs& w,
                                 double2* plane_sums, hipStream_t s) {
     const Team g = team_of(p, t, true, 1);
-    launch_clear(p, g, part, s);
-    const dim3 grid((unsigned)(p.units * g.blocks));
+    launch_clear(p, g, w, s);
+    const int64_t blocks = p.units * g.blocks;
+    const dim3 grid((unsigned)blocks);
     bsel((a.flags & SOAR_GN_SILU) != 0, [&](auto S) {
         bsel((a.flags & SOAR_GN_RESIDUAL) != 0, [&](auto R) {
             k_team_bwd<S(), R()><<<grid, kTeamThreads, 0, s>>>(
                 a.dy, a.x, a.gamma, a.beta, a.mean, a.rstd, a.mean_lo, a.dx, a.dgamma, a.dbeta,
-                plane_sums, reinterpret_cast<u64*>(part), g);
+                plane_sums, w, g);
+            k_team_bwd_rest<S(), R()><<<rest_grid(blocks), kTeamThreads, 0, s>>>(
+                a.dy, a.x, a.gamma, a.beta, a.mean, a.rstd, a.mean_lo, a.dx, a.dgamma, a.dbeta,
+                plane_sums, w, g, blocks);
         });
     });
     return hipGetLastError();

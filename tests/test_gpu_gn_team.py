@@ -1,7 +1,7 @@
 """GroupNorm(+SiLU) with the unit kept on chip between the passes, against
 float64 and against the two-launch path over the forms that both accept, and
-with every wait ending at once (each block then computes the sums it misses
-itself)."""
+with every wait ending at once: each block then leaves its share to the launch
+after unless the sums are there by then, or leaves it in any case."""
 import numpy as np
 import pytest
 import torch
@@ -93,6 +93,19 @@ def test_team_matches_float64_and_two_launches(gpu, wait_us, case):
         # two of fp32 apart
         assert (a - b).abs().max() <= 4 * 2.0 ** -23 * scale, what
         assert (a.double() - t).abs().max() <= 1e-5 * scale, what
+
+
+@pytest.mark.parametrize("case", CASES)
+def test_every_block_may_leave(gpu, wait_us, case):
+    """No block gets its unit's sums in time, so all of the output comes from
+    the launch after: bit for bit a team's, every gradient added once."""
+    N, C, HW, G, silu, residual, affine = case
+    x, dy, gamma, beta = tensors(N, C, HW, affine)
+    args = (gpu, x, dy, gamma, beta, G, silu, residual)
+    want = both(*args)
+    wait_us(-2)
+    for a, b, what in zip(both(*args), want, ("y", "mean", "rstd", "dx", "dgamma", "dbeta")):
+        assert torch.equal(a, b), what
 
 
 def test_team_leaves_overlapping_outputs_alone(gpu):
