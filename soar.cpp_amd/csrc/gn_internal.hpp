@@ -102,7 +102,7 @@ struct Tuning {
     int64_t dw_cba_min = 16384;  // depthwise CBA backward: samples x pixels
                                  // from which the fused kernel runs (0:
                                  // never)
-    int64_t team_wait_us = 200;  // gn_team.hip: microseconds a block waits for
+    int64_t team_wait_us = 100;  // gn_team.hip: microseconds a block waits for
                                  // its team's sums before it leaves its share
                                  // to the launch after; or kTeamOff, kTeamLeave
     int64_t pw_cba_blocks = 256;  // and the blocks its pixel chunks aim for

@@ -11,20 +11,20 @@
 // What bounds it: memory, in phases.  A team loads, waits and stores, and
 // while it waits only the next team's blocks load; a copy from registers in
 // such phases takes 375-390 us per 2 GiB moved, a streaming copy 332.  So
-// teams are kept small against the chip (several in flight) where the unit
-// allows.  Measured with SiLU, two launches -> one (forward; backward; backward
-// without SiLU), us:
-//   32 x 512^2, 8 groups    21.6 -> 16.5; 33.6 -> 23.1; 32.1 -> 21.7
-//   64 x 512^2, 16          36.8 -> 26.0; 59.2 -> 43.8; 57.4 -> 39.9
-//   32 x 1024^2, 8          66.1 -> 51.3; 104 -> 94;    103 -> 85
-//   64 x 1024^2, 16         125 -> 101;   204 -> 189;   203 -> 168
-//   2 x 128 x 1024^2, 32    490 -> 401;   815 -> 761;   817 -> 667
-//   64 x 2048^2, 16         491 -> 436-458; (too large)
-// Held on chip per block: 512 threads at 128 VGPRs, two blocks per CU, so up
-// to 32 (64) floats of x per thread in registers and 16 more in LDS forward,
-// 32 of x and 32 of dy backward.  (Backward with a further chunk in LDS, for
-// units of 64 MB, gained 4% and needed the whole chip to itself; reading x
-// again instead of holding it was slower than two launches.)
+// teams are kept small against the chip (several in flight).  Measured with
+// SiLU, two launches -> one, forward; backward, us:
+//   48 x 512^2, 8 groups         30.6 -> 23.0; 45.7 -> 37.0
+//   64 x 512^2, 16               36.6 -> 27.1; 57.6 -> 43.9
+//   16 x 1024^2, 8               37.5 -> 27.0; 56.9 -> 45.1
+//   24 x 1024^2, 4               52.2 -> 36.9; (too large)
+//   32 x 1024^2, 8               65.9 -> 51.5; (too large)
+//   2 x 64 x 1024^2, 32          246 -> 191;   406 -> 330
+//   2 x 128 x 1024^2, 32, +x     483 -> 386;   (too large)
+// Held on chip per block: 512 threads at 128 VGPRs, two blocks per CU, so 64
+// floats of x per thread in registers and 32 more in LDS forward, 32 of x and
+// 32 of dy backward.  (Backward with a further chunk in LDS gained 4% and
+// needed the whole chip to itself; reading x again instead of holding it was
+// slower than two launches.)
 //
 // Every chunk (8192 floats of a plane, 256 threads of 8 vectors) and output
 // uses the arithmetic of k_stats / k_apply / k_bwd_reduce / k_bwd_dx in the
@@ -49,10 +49,11 @@
 // unit in the slots, reads the unit again and writes it, the second pass of
 // two launches; the bits are the same.  No loop ends by another block's
 // store, and once a block of the call has left, the others do not wait
-// either, so a call that meets other work costs one limit more than two
-// launches.  (A marked unit is read after blocks of it wrote theirs, which
-// is why outputs that overlap inputs take the two launches.)  Where nothing
-// is marked the launch ends at once.
+// either: a call that meets other work costs its limit once (with every
+// block leaving, forward; backward: 64 x 512^2 55.8; 88.9 us, 32 x 1024^2
+// forward 96).  A marked unit is read after blocks of it wrote theirs, which
+// is why outputs that overlap inputs take the two launches.  Where nothing is
+// marked the launch ends at once (1.2 us).
 #include <algorithm>
 #include <atomic>
 #include <type_traits>
@@ -77,23 +78,29 @@ constexpr int kTeamThreads = 512;
 constexpr int kHalf = 256;     // threads of a half-block, which walks whole chunks
 constexpr int kVec = 8;        // vectors of a chunk per thread
 constexpr int kTeamChunk = 4 * kVec * kHalf;  // 8192 floats
-constexpr int kMaxItems = 1024;                // per unit
 constexpr int kMaxCpg = 128;                  // channels per unit
-// Blocks of a team, of the 512 that 256 CUs hold: with fewer, the team after
-// it is already loading, and work of other streams on some CUs does not keep
-// a team from running together.
-constexpr int kMaxTeam = 400;
-// Chunks of the tensor (24 MB).  Below, both ways live in the caches and the
-// launches decide, of which this way has one more each way and dgamma's with
-// several samples.  Forward; backward, us, two launches -> one: 256 chunks
-// 9.3 -> 10.1; 12.1 -> 12.8, 512 (64 x 256^2) 11.4 -> 11.4; 19.5 -> 14.9 (but
-// 20.4 -> 21.3 with residual and two samples), 768 (96 x 256^2) 17.0 -> 13.2;
-// 26.5 -> 20.2, 1024 (32 x 512^2) 21.1 -> 15.8; 33.1 -> 22.3.
-constexpr int64_t kTeamMinChunks = 768;
+// Blocks of a team: a quarter of the 512 that 256 CUs hold.  Calls of other
+// streams take their part of every CU, and a team that is only partly there
+// waits for its limit; the part that is left for it must hold it.  Two streams
+// of the same calls, us a pair, in two launches -> with teams of 128; 192;
+// 256; 342 blocks (a limit of 50-100 us): 1012 -> 861 (forward, 2 x 128 x
+// 1024^2), 100 -> 91 (backward, 16 x 1024^2); 149 -> 151; 206 -> 317 and 1629
+// -> 2755 (backward, 32 and 2 x 128 x 1024^2; alone such a team gains 10%).
+// Three streams: 0.92-0.99 of two launches' time at 128, 1.4 at 192; four up
+// to 1.2 at 128, since blocks then leave.
+constexpr int kMaxTeam = 128;
+// Chunks of the tensor, forward (48 MB) and backward (24 MB).  Below, both
+// ways live in the caches and the launches decide, of which this way has one
+// more each way (three, at 2.4 us each for the host) and dgamma's with several
+// samples.  Two launches -> one, us, replayed from a graph and called one by
+// one: forward of 768 chunks 18.0 -> 15.3 and 18.9 -> 21.7, 1024 21.3 -> 17.8
+// and 21.7 -> 20.6 (two streams 38.4 -> 42.2), 1536 30.6 -> 23.0; backward of
+// 768 27.6 -> 20.5, 1024 33.8 -> 23.8.
+constexpr int64_t kTeamMinFwd = 1536, kTeamMinBwd = 768;
 // Chunks up to which a backward with residual and SiLU comes here (64 MB): its
 // dy stays held and the SiLU's derivative is formed again after the wait.  Two
-// launches -> one, us: 32 x 512^2 32.8 -> 26.0, 64 x 512^2 60.2 -> 50.0, 32 x
-// 1024^2 104.0 -> 102.6, 64 x 1024^2 203 -> 206, 2 x 128 x 1024^2 812 -> 830.
+// launches -> one, us: 64 x 512^2 57.9 -> 43.7; larger, with more spilled
+// registers than now, 64 x 1024^2 203 -> 206, 2 x 128 x 1024^2 812 -> 830.
 // (gamma r dz + dy in dy's place instead: 73 spilled registers, 1199.)
 constexpr int64_t kTeamMaxResChunks = 2048;
 constexpr u64 kUnset = ~0ull;
@@ -740,7 +747,7 @@ Team team_of(const Plan& p, const Tuning& t, bool bwd, int depth) {
 bool team_fits(const Plan& p, const Tuning& t, const Team& g) {
     return t.team_wait_us != kTeamOff && p.chunk == kTeamChunk && p.HW % 4 == 0 && p.cpg <= kMaxCpg &&
            p.cpg * p.cpp <= (int64_t)1 << 20 && p.units * p.cpg * p.cpp < (int64_t)1 << 30 &&
-           g.items <= kMaxItems && g.blocks <= kMaxTeam * device_cus() / 256;
+           g.blocks <= kMaxTeam * device_cus() / 256;
 }
 
 void launch_clear(const Plan& p, const Team& g, const TeamWs& w, hipStream_t s) {
@@ -764,26 +771,24 @@ bool overlap(const Plan& p, const float* a, const float* b) {
 
 }  // namespace
 
-// Chunks per half-block, 0: two launches.  One if the tensor's blocks are at
-// most two waves of the chip (64 x 512^2, 2048 chunks: 23.6 us at two chunks,
-// 26.0 at one), else two: half the slots to look at.  Three (LDS) only for
-// units that need it (64 x 2048^2: 448 us; with 512 blocks of two, 436, but
-// such a team needs the whole chip).
+// Chunks per half-block, 0: two launches.  Two, in registers (fewer slots to
+// look at than with one); three, with LDS, only for units that need it (more
+// than 512 chunks).
 int team_fwd_depth(const Plan& p, const Tuning& t, const FwdArgs& a) {
     const int64_t chunks = p.units * p.cpg * p.cpp;
     if (a.res || !aligned(a.x) || !aligned(a.y) || overlap(p, a.x, a.y)) return 0;
-    if (chunks < kTeamMinChunks) return 0;
-    for (int depth = chunks <= 4 * device_cus() ? 1 : 2; depth <= 3; ++depth)
+    if (chunks < kTeamMinFwd) return 0;
+    for (int depth = 2; depth <= 3; ++depth)
         if (team_fits(p, t, team_of(p, t, false, depth))) return depth;
     return 0;
 }
 
-// Units of at most 800 chunks (26 MB) backward: the size of a team.
+// Units of at most 256 chunks (8 MB) backward: the size of a team.
 bool team_bwd_fits(const Plan& p, const Tuning& t, const BwdArgs& a) {
     const bool res_silu = (a.flags & SOAR_GN_RESIDUAL) && (a.flags & SOAR_GN_SILU);
     return a.dx && !(a.flags & SOAR_GN_ACCUMULATE_DX) && aligned(a.x) && aligned(a.dy) &&
            aligned(a.dx) && !overlap(p, a.x, a.dx) && !overlap(p, a.dy, a.dx) &&
-           p.units * p.cpg * p.cpp >= kTeamMinChunks &&
+           p.units * p.cpg * p.cpp >= kTeamMinBwd &&
            !(res_silu && p.units * p.cpg * p.cpp > kTeamMaxResChunks) &&
            team_fits(p, t, team_of(p, t, true, 1));
 }
@@ -803,11 +808,10 @@ hipError_t launch_team_forward(const Plan& p, const Tuning& t, const FwdArgs& a,
             using Z = std::integral_constant<int, 0>;
             using I1 = std::integral_constant<int, 1>;
             using I2 = std::integral_constant<int, 2>;
-            switch (depth) {
-                case 1: go(I1{}, Z{}); break;
-                case 2: go(I2{}, Z{}); break;
-                default: go(I2{}, I1{});
-            }
+            if (depth == 2)
+                go(I2{}, Z{});
+            else
+                go(I2{}, I1{});
             k_team_fwd_rest<S(), R()><<<rest_grid(blocks), kTeamThreads, 0, s>>>(
                 a.x, a.gamma, a.beta, a.y, a.mean, a.rstd, a.mean_lo, w, g, a.eps, blocks, depth);
         });

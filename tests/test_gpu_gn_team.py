@@ -2,7 +2,8 @@
 float64 and against the two-launch path over the forms that both accept, and
 with every wait ending at once: each block then leaves its share to the launch
 after unless the sums are there by then, or leaves it in any case."""
-import numpy as np
+import time
+
 import pytest
 import torch
 
@@ -13,16 +14,21 @@ pytestmark = pytest.mark.gpu
 CASES = [
     # (N, C, HW, G, silu, residual, affine)
     (1, 768, 8192, 8, True, False, True),        # one chunk per plane, 768 in all: the least
-    (2, 192, 8196, 4, True, True, True),         # a last chunk of one vector
-    (3, 96, 25600, 8, False, False, True),       # plain GroupNorm, a ragged last chunk
-    (1, 32, 262144, 32, True, False, False),     # one plane per unit, no affine
-    (2, 64, 65536, 8, False, True, True),
+    (2, 768, 8192, 8, True, False, True),        # 1536: the least forward
+    (4, 192, 8196, 4, True, True, True),         # a last chunk of one vector
+    (4, 96, 25600, 8, False, False, True),       # plain GroupNorm, a ragged last chunk
+    (2, 32, 262144, 32, True, False, False),     # one plane per unit, no affine
+    (3, 64, 65536, 8, False, True, True),
     (2, 128, 73728, 16, True, True, True),       # forward only: backward above 2048 chunks
-    (1, 512, 8196, 4, True, False, True),        # 128 planes per unit, the most
-    (1, 96, 102400, 16, True, False, True),      # forward: two chunks per half-block
-    (1, 6, 4194304, 2, True, False, True),       # three (LDS); backward too large
-    (3, 99, 28672, 3, True, False, True),        # odd channels per unit
+    (2, 512, 8196, 4, True, False, True),        # 128 planes per unit, the most
+    (2, 96, 102400, 16, True, False, True),
+    (1, 6, 2097152, 2, True, False, True),       # forward: three chunks per half-block (LDS)
+    (4, 99, 28672, 3, True, False, True),        # odd channels per unit
 ]
+
+
+def chunks(N, C, HW):
+    return N * C * -(-HW // 8192)
 
 
 def tensors(N, C, HW, affine, seed=3):
@@ -78,8 +84,8 @@ def test_team_matches_float64_and_two_launches(gpu, wait_us, case):
     torch.cuda.synchronize()
     names = {p["kernel"] for p in gpu.prof_summary()}
     gpu.prof_enable(False)
-    assert any("team_fwd" in n for n in names), names
-    held = C // G * HW <= 2 ** 22 and not (silu and residual and N * C * HW > 2 ** 24)
+    assert any("team_fwd" in n for n in names) == (chunks(N, C, HW) >= 1536), names
+    held = chunks(1, C // G, HW) <= 256 and not (silu and residual and chunks(N, C, HW) > 2048)
     assert any("team_bwd" in n for n in names) == held, names
     wait_us(-1)
     two = both(*args)
@@ -110,7 +116,7 @@ def test_every_block_may_leave(gpu, wait_us, case):
 
 def test_team_leaves_overlapping_outputs_alone(gpu):
     """In place, the two launches run, as they always did."""
-    x, dy, gamma, beta = tensors(1, 128, 65536, True)
+    x, dy, gamma, beta = tensors(2, 128, 65536, True)
     y, st = gpu.gn_silu_forward(x, gamma, beta, 8, eps=EPS)
     inplace = x.clone()
     gpu.gn_silu_forward(inplace, gamma, beta, 8, eps=EPS, y=inplace)
@@ -122,11 +128,11 @@ def test_team_leaves_overlapping_outputs_alone(gpu):
 
 
 def test_team_graph_replays(gpu):
-    x, dy, gamma, beta = tensors(2, 64, 65536, True)
-    ws = gpu.workspace(2, 64, 65536, 8)
+    x, dy, gamma, beta = tensors(3, 64, 65536, True)
+    ws = gpu.workspace(3, 64, 65536, 8)
     want = both(gpu, x, dy, gamma, beta, 8, True, False)
     y, dx = torch.empty_like(x), torch.empty_like(x)
-    st = [torch.empty(16, device="cuda") for _ in range(3)]
+    st = [torch.empty(24, device="cuda") for _ in range(3)]
     dg, db = torch.zeros(64, device="cuda"), torch.zeros(64, device="cuda")
 
     def step():
@@ -170,3 +176,49 @@ def test_team_on_two_streams(gpu):
     for g in got:
         for a, b in zip(g, want):
             assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("shape", [(1, 16, 1048576, 8), (1, 32, 1048576, 8), (1, 24, 1048576, 4),
+                                   (1, 64, 4194304, 16)])
+@pytest.mark.parametrize("backward", [False, True])
+def test_streams_cost_no_more_than_two_launches(gpu, wait_us, shape, backward):
+    """Two streams' calls at once take no longer than where every call reads
+    its tensor twice (bar: a third more, for timing).  Where a team needed more
+    than half of the chip, both streams' teams stood in each other's way: 2 to
+    20 times as long."""
+    N, C, HW, G = shape
+    calls = []
+    for i in range(2):
+        x, dy, gamma, beta = tensors(N, C, HW, True, seed=i)
+        y, dx, ws = torch.empty_like(x), torch.empty_like(x), gpu.workspace(N, C, HW, G)
+        st = [torch.empty(N * G, device="cuda") for _ in range(3)]
+        dg, db = torch.zeros(C, device="cuda"), torch.zeros(C, device="cuda")
+        _, s = gpu.gn_silu_forward(x, gamma, beta, G, y=y, mean=st[0], rstd=st[1], mean_lo=st[2],
+                                   ws=ws)
+        # (default arguments: each call keeps its own tensors)
+        if backward:
+            calls.append(lambda dy=dy, x=x, ga=gamma, be=beta, s=s, dx=dx, dg=dg, db=db, ws=ws:
+                         gpu.gn_silu_backward(dy, x, ga, be, s, G, dx=dx, dgamma=dg, dbeta=db,
+                                              ws=ws))
+        else:
+            calls.append(lambda x=x, ga=gamma, be=beta, y=y, st=st, ws=ws: gpu.gn_silu_forward(
+                x, ga, be, G, y=y, mean=st[0], rstd=st[1], mean_lo=st[2], ws=ws))
+    streams = [torch.cuda.Stream() for _ in calls]
+
+    def run():
+        torch.cuda.synchronize()
+        t0 = time.perf_counter()
+        for _ in range(10):
+            for s, call in zip(streams, calls):
+                with torch.cuda.stream(s):
+                    call()
+        torch.cuda.synchronize()
+        return time.perf_counter() - t0
+
+    default = gpu.tune_get(gpu.TUNE_TEAM_WAIT_US)
+    best = {}
+    for wait in (default, -1) * 4:
+        wait_us(wait)
+        t = run()
+        best[wait] = min(t, best.get(wait, t))
+    assert best[default] <= 1.33 * best[-1], best
