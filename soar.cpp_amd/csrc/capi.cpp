@@ -596,9 +596,10 @@ int pw_conv_gn_forward(const float* x, const float* weight, const float* bias,
     const hipStream_t s = static_cast<hipStream_t>(stream);
     soar::gn::PwArgs pa{x, weight, bias, z};
     Plan q;
-    if (soar::gn::pw_use_small(N, C_out, C_in, HW, t.pw_small) &&
-        soar::gn::make_plan(N, C_out, HW, G, t, &q)) {
-        // Small planes: the SIMT convolution (no statistics epilogue), then
+    if (soar::gn::make_plan(N, C_out, HW, G, t, &q) &&
+        soar::gn::pw_use_small_norm(N, C_out, C_in, HW, t.pw_small,
+                                    soar::gn::forward_is_small(q, t))) {
+        // Small planes: the convolution without a statistics epilogue, then
         // the GroupNorm forward over z with its own plan.
         if ((rc = check_ws(q, workspace, workspace_bytes))) return rc;
         hipError_t e = soar::gn::launch_pw_conv(pa, N, C_in, C_out, HW, p.chunk, nullptr, false,

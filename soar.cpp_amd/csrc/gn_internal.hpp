@@ -284,7 +284,9 @@ hipError_t launch_pw_conv(const PwArgs& a, int64_t N, int64_t C_in, int64_t C_ou
                           const char* name = nullptr, bool wt = false);
 // The block-tiled convolution of wide layers (pw_gemm.hip): M output rows,
 // K input rows; `trans`: weights [K][M].  chunk as for launch_pw_conv.
+// pw_gemm_loses: pw_use_small's kernel is faster.
 bool pw_gemm_use(int64_t N, int64_t K, int64_t M, int64_t HW);
+bool pw_gemm_loses(int64_t N, int64_t K, int64_t M, int64_t HW, bool norm);
 hipError_t launch_pw_gemm(const PwArgs& a, int64_t N, int64_t K, int64_t M, int64_t HW,
                           int64_t chunk, double2* part, bool accumulate, bool trans,
                           hipStream_t s);
@@ -309,6 +311,11 @@ size_t pw_kz_max_bytes(int64_t N, int64_t C_out, int64_t HW, int64_t chunk, int 
 // terms each): at most `small` multiply-adds, and offsets inside a sample
 // fit in 32 bits.
 bool pw_use_small(int64_t N, int64_t M, int64_t K, int64_t HW, int64_t small);
+// The same before a GroupNorm that would otherwise take the convolution's
+// statistics; small_units: one launch over z does all of it.  (The
+// convolution itself is then pw_use_small's choice.)
+bool pw_use_small_norm(int64_t N, int64_t M, int64_t K, int64_t HW, int64_t small,
+                       bool small_units);
 
 // Backward of the pointwise convolution: dx = W^T dz (written, or added
 // with `accumulate_dx`), dw += sum dz x^T, db += sum dz; any output may be

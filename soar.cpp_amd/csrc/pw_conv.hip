@@ -1654,9 +1654,19 @@ bool pw_use_small_wgrad(int64_t N, int64_t C_in, int64_t C_out, int64_t HW, int6
 // launches): the SIMT kernel wins up to about 2^25 multiply-adds (256 ->
 // 128 channels at 1024 pixels: 11 vs 19 us; 64 -> 128 at 4096: 10 vs 13
 // us), ties at 2^26 and loses above (512 -> 256 at 1024: 34 vs 28 us; 128
-// -> 256 at 4096: 35 vs 16 us).
+// -> 256 at 4096: 35 vs 16 us).  Against the block-tiled kernel, where that
+// runs: pw_gemm_loses.
 bool pw_use_small(int64_t N, int64_t M, int64_t K, int64_t HW, int64_t small) {
-    return small > 0 && pw_small_fits(N, M, K, HW) && !pw_gemm_use(N, K, M, HW) &&
+    return small > 0 && pw_small_fits(N, M, K, HW) &&
+           (!pw_gemm_use(N, K, M, HW) || pw_gemm_loses(N, K, M, HW, false)) &&
+           (double)N * (double)M * (double)K * (double)HW <= (double)small;
+}
+
+bool pw_use_small_norm(int64_t N, int64_t M, int64_t K, int64_t HW, int64_t small,
+                       bool small_units) {
+    if (!pw_gemm_use(N, K, M, HW)) return pw_use_small(N, M, K, HW, small);
+    return small > 0 && pw_small_fits(N, M, K, HW) && small_units &&
+           pw_gemm_loses(N, K, M, HW, true) &&
            (double)N * (double)M * (double)K * (double)HW <= (double)small;
 }
 
@@ -1854,7 +1864,8 @@ hipError_t launch_pw_conv(const PwArgs& a, int64_t N, int64_t C_in, int64_t C_ou
         return launch_pw_small(a.x, a.w, a.bias, a.z, N, C_in, C_out, HW, false, accumulate, s,
                                name ? name : "pw_conv_small");
     if (pw_gemm_use(N, C_in, C_out, HW)) {
-        const int tok = prof_begin(s, name ? name : (part ? "pw_conv_gn_stats" : "pw_conv"));
+        const int tok = prof_begin(s, wt ? "pw_conv_dgrad_tiled"
+                                         : (part ? "pw_conv_gn_stats_tiled" : "pw_conv_tiled"));
         const hipError_t e = launch_pw_gemm(a, N, C_in, C_out, HW, chunk, part, accumulate, wt, s);
         prof_end(s, tok);
         return e;
@@ -2067,7 +2078,7 @@ hipError_t launch_pw_backward(const PwBwdPlan& p, const PwBwdArgs& a, int64_t N,
         const bool fast = (HW % 4 == 0) && ((uintptr_t)a.dz % 16 == 0) &&
                           ((uintptr_t)a.x % 16 == 0);
         const dim3 grid((unsigned)(p.tiles_co * p.tiles_ci), (unsigned)p.Gb);
-        int tok = prof_begin(s, "pw_conv_wgrad");
+        int tok = prof_begin(s, p.gemm_dw ? "pw_conv_wgrad_tiled" : "pw_conv_wgrad");
         if (p.gemm_dw) {
             const hipError_t e = launch_pw_gemm_wgrad(a.dz, a.x, part_w, a.db ? part_b : nullptr,
                                                       N, C_in, C_out, HW, p.chunk_b, s);

@@ -519,10 +519,34 @@ static bool gemm_fits(int64_t N, int64_t K, int64_t M, int64_t HW) {
 // split K (512 -> 256 at 1024 pixels, 32 tiles: 31.4 here, 20.2 us there;
 // 256 -> 128 at 4096, 64 tiles: 22.4 and 21.6 us; 512 -> 256 at 4096, 128
 // tiles: 34.1 and 37.8 us).
+static int64_t gemm_tiles(int64_t N, int64_t M, int64_t HW) {
+    return N * ((HW + kGp - 1) / kGp) * ((M + kGm - 1) / kGm);
+}
+
 bool pw_gemm_use(int64_t N, int64_t K, int64_t M, int64_t HW) {
     if (M < 48 || K < 48 || !gemm_fits(N, K, M, HW)) return false;
-    const int64_t tiles = N * ((HW + kGp - 1) / kGp) * ((M + kGm - 1) / kGm);
+    const int64_t tiles = gemm_tiles(N, M, HW);
     return tiles >= 32 && K <= 4 * tiles;
+}
+
+// Whether k_pw_small, within its own limit, is still faster.  Its time goes
+// with the multiply-adds; here a tile that is partly filled (a plane of fewer
+// than 128 pixels) takes as long as a full one, and the time goes with the K
+// steps and, beyond about two blocks per CU, with the tiles.  us, k_pw_small /
+// here: 512 -> 512 channels, 32 samples of 1 pixel 7.1 / 30.1; 256 -> 256, 16
+// of 4 3.5 / 13.6; 64 -> 64, 32 of 49 4.5 / 7.0; 128 -> 128, 16 of 64 6.3 /
+// 8.5 and 32 of 49 (2^24.6 multiply-adds) 11.2 / 10.2; 256 -> 256, 128 of 4
+// 10.2 / 14; input gradients 192 <- 384, 48 of 9 20 / 16, 512 <- 512, 128 of 1
+// 11 / 74.  Over 700 calls of at most 2^25 multiply-adds the line's choice
+// takes 0.3% longer than the faster one on average and 20% at most; the tile
+// everywhere 58%, at most 6.8 times as long.  `norm`: a GroupNorm of small
+// units follows, which takes one launch over z but two on the tile's
+// statistics (16 x 64 -> 64 at 16 x 16: 10.2 / 11.4, without it 6.2 / 6.0).
+bool pw_gemm_loses(int64_t N, int64_t K, int64_t M, int64_t HW, bool norm) {
+    const double steps = (double)((K + kGk - 1) / kGk);
+    const double waves = std::max(1.0, (double)gemm_tiles(N, M, HW) / 512.0);
+    const double macs = (double)N * (double)K * (double)M * (double)HW;
+    return macs <= ((norm ? 11.0 : 7.0) + 3.5 * steps * waves) * 1048576.0;
 }
 
 // 192 -> 384 channels at 128^2 pixels: forward with statistics 49.5 -> 23.9

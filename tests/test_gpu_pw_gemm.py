@@ -102,3 +102,38 @@ def test_pw_gemm_non_finite_operands(gpu, value):
             assert np.isfinite(host(dw)[rest]).all()
     # columns and rows that nothing non-finite reaches
     np.testing.assert_allclose(host(dw)[:70, 6:], host(dwc)[:70, 6:], rtol=1e-3, atol=1e-3)
+
+
+@pytest.mark.parametrize("shape, forward, fused, dgrad", [
+    # (N, C_in, C_out, HW), whether the block-tiled kernel runs: 32 tiles of
+    # 128 pixels and more each
+    ((32, 512, 512, 1), False, False, False),    # 1 pixel of a tile: 7 against 30 us
+    ((16, 256, 256, 4), False, False, False),
+    ((32, 64, 64, 49), False, False, False),
+    ((8, 64, 64, 400), False, False, False),     # 12.5 * 2^20 multiply-adds, the line at 14
+    ((16, 64, 64, 256), True, False, True),      # 16 * 2^20; the fused form's line at 18
+    ((32, 128, 128, 49), True, False, True),     # 24.5 * 2^20, the lines at 21 and 25
+    ((128, 512, 512, 1), False, False, False),   # 2^25, 1024 tiles
+    ((1, 64, 64, 4096), True, True, True),       # units of more than 16384: statistics fused
+    ((1, 128, 256, 4096), True, True, True),
+])
+def test_pw_gemm_leaves_small_layers(gpu, shape, forward, fused, dgrad):
+    import torch
+    N, C_in, C_out, HW = shape
+    x, w, b, dz = (dev(v) for v in data(5, *shape))
+    ga, be = torch.ones(C_out, device="cuda"), torch.zeros(C_out, device="cuda")
+
+    def kernels(fn):
+        gpu.prof_summary()  # drop earlier records
+        gpu.prof_enable(True)
+        fn()
+        torch.cuda.synchronize()
+        names = {p["kernel"] for p in gpu.prof_summary()}
+        gpu.prof_enable(False)
+        return names
+
+    assert ("pw_conv_tiled" in kernels(lambda: gpu.pw_conv_forward(x, w, b))) == forward
+    got = kernels(lambda: gpu.pw_conv_gn_silu_forward(x, w, b, ga, be, 8))
+    assert ("pw_conv_gn_stats_tiled" in got) == fused, got
+    got = kernels(lambda: gpu.pw_conv_backward(dz, x, w, want_dw=False, want_db=False))
+    assert ("pw_conv_dgrad_tiled" in got) == dgrad, got
