@@ -2,21 +2,29 @@
 //
 // gfx950's bf16 matrix instructions run at 16 times the rate of its fp32
 // ones.  An fp32 value is split into three bf16 parts, x = h + m + l, each
-// the round-to-nearest bf16 of what the parts before it leave: |m| <= 2^-9
-// |x|, |l| <= 2^-18 |x|, and what l leaves is at most 2^-27 |x|.  A product
-// then takes the six part products down to 2^-18 of it,
+// the round-to-nearest bf16 (eight significant bits) of what the parts before
+// it leave: |m| <= 2^-8 |x|, |l| <= 2^-17 |x|, and l leaves nothing.  A
+// product then takes the six part products down to 2^-17 of it,
 //   h h' + (h m' + m h') + (m m' + h l' + l h'),
 // each exact in fp32 and added in fp32 by the matrix core; the three left
-// out and the splits' remainders are together at most 2^-25 |x x'|, half an
-// fp32 rounding of the product itself.  So the result has the error of an
-// fp32 dot product, at 6/16 of its matrix time plus the splits.
+// out are together at most 2^-24 |x x'|, as much as rounding the product to
+// fp32 (on average less: a sum of many products is nearer to exact than an
+// fp32 one, mma_step; a single product's error can be twice as large).  It
+// takes 6/16 of the fp32 matrix time plus the splits.
 //
-// Non-finite inputs: an infinity (or a finite value that rounds to one as
-// bf16, |x| >= 2^128 (1 - 2^-9)) leaves a NaN remainder, so every output it
-// reaches comes out non-finite.  The kernels test their accumulators and
-// run a tile that has a non-finite one again on the fp32 instructions, so
-// infinities and NaN come out as fp32 products and sums give them.  (Parts
-// below 2^-126 are flushed: an absolute error below 2^-126 |x'|.)
+// Range.  The parts are those of 2^16 x (kBf3Up): fp32's last bit is 2^-149,
+// bf16's 2^-133 (the conversions and the matrix cores keep denormals), so
+// the split is exact for every x; unscaled, it lost bits from 2^-109 down.
+// Sums come out 2^32 times as large and are scaled back by kBf3Down.  The
+// scale costs 2-4%: 192 -> 384 channels at 128^2 pixels forward 22.4 -> 23.0,
+// input gradient 25.8 -> 26.8, weight gradient with its finish 34.0 -> 35.0 us.
+//
+// Non-finite inputs: an infinity (or a finite value that the scale takes
+// there, |x| >= 2^112) leaves a NaN remainder, so every output it reaches
+// comes out non-finite, as does one above 2^96.  The kernels test their
+// accumulators and run a tile that has a non-finite one again on the fp32
+// instructions, so infinities, NaN and large values come out as fp32 products
+// and sums give them.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -33,8 +41,10 @@ struct Bf3 {
     u4 p[3];  // h, m, l: pairs of bf16 values
 };
 
-// The parts of eight values: per pair three packed conversions and four
-// unpacked subtractions, eleven instructions.  (A remainder as one bf16 dot
+constexpr float kBf3Up = 0x1p16f, kBf3Down = 0x1p-32f;
+
+// The parts of eight values, scaled: per pair two products, three packed
+// conversions and four unpacked subtractions, thirteen instructions.  (A remainder as one bf16 dot
 // product with (-1, 0) takes seven, but v_dot2_f32_bf16 does not run beside
 // the matrix instructions of the SIMD as these do: 24 MFMAs with 144 of
 // either took 1503 ns against 876-921 for two waves of a SIMD, 783 ns for
@@ -42,7 +52,10 @@ struct Bf3 {
 __device__ __forceinline__ Bf3 bf3_split(float v0, float v1, float v2, float v3, float v4,
                                          float v5, float v6, float v7) {
     typedef float f2 __attribute__((ext_vector_type(2)));
-    f2 v[4] = {{v0, v1}, {v2, v3}, {v4, v5}, {v6, v7}};
+    f2 v[4] = {{v0 * kBf3Up, v1 * kBf3Up},
+               {v2 * kBf3Up, v3 * kBf3Up},
+               {v4 * kBf3Up, v5 * kBf3Up},
+               {v6 * kBf3Up, v7 * kBf3Up}};
     Bf3 o;
 #pragma unroll
     for (int p = 0; p < 3; ++p) {

@@ -302,8 +302,11 @@ __global__ __launch_bounds__(256, 3) void k_pw_gemm(
         }
         acc[0] += lo[0];
         acc[1] += lo[1];
-        if (any_nonfinite(acc)) {
-            // an infinity or NaN among the operands: again on fp32 instructions
+        if (!any_nonfinite(acc)) {
+            acc[0] *= kBf3Down;
+            acc[1] *= kBf3Down;
+        } else {
+            // an infinity, NaN or large value: again on fp32 instructions
             clear(acc);
             const int64_t row = min<int64_t>(slot_row(32 * wm + j), M - 1);
             for (int64_t k = 0; k < K; k += 2) {
@@ -455,8 +458,11 @@ __global__ __launch_bounds__(256, 3) void k_pw_gemm_wgrad(
     }
     acc[0] += lo[0];
     acc[1] += lo[1];
-    if (any_nonfinite(acc)) {
-        // an infinity or NaN among the operands: again on fp32 instructions
+    if (!any_nonfinite(acc)) {
+        acc[0] *= kBf3Down;
+        acc[1] *= kBf3Down;
+    } else {
+        // an infinity, NaN or large value: again on fp32 instructions
         clear(acc);
         for (int64_t p = px0; p < pend; p += 2) {
             const int64_t pp = p + h;

@@ -38,7 +38,7 @@ def data(seed, N, C_in, C_out, HW):
 
 
 def check(got, truth, bound, what):
-    ratio = np.abs(np.asarray(got, np.float64) - truth) / (bound + 1e-30)
+    ratio = np.abs(np.asarray(got, np.float64) - truth) / np.maximum(bound, 2.0 ** -149)
     assert ratio.max() <= 1.0, f"{what}: {ratio.max():.2f} of the bound"
 
 
@@ -69,6 +69,30 @@ def test_pw_gemm_matches_float64(gpu, oracle, shape):
     bw = 1026 * U32 * np.einsum("nop,ncp->oc", np.abs(D), np.abs(X), optimize=True)
     check(host(dw_), tw, bw, "dw")
     check(host(db_), D.sum((0, 2)), 1026 * U32 * np.abs(D).sum((0, 2)), "db")
+
+
+@pytest.mark.parametrize("ex, ew", [(-112, 0), (-122, 0), (0, -118), (-112, 100), (100, -120),
+                                    (-60, -60), (60, 50), (90, 20), (115, -100)])
+def test_pw_gemm_operands_of_any_size(gpu, ex, ew):
+    """Operands anywhere in fp32's range keep their 24 bits, however small the
+    parts that they split into: the bar of the other tests at every scale
+    (and, where a product is below 2^-126, fp32's spacing there)."""
+    N, C_in, C_out, HW = 1, 64, 96, 4096
+    x, w, _, dz = data(13, N, C_in, C_out, HW)
+    # exact scales, powers of two
+    x, dz, w = (np.ldexp(v, e).astype(np.float32) for v, e in ((x, ex), (dz, ex), (w, ew)))
+    X, W, D = x.astype(np.float64), w.astype(np.float64), dz.astype(np.float64)
+    tiny = 2.0 ** -149
+    z = gpu.pw_conv_forward(dev(x), dev(w))
+    check(host(z), W @ X, (C_in + 2) * (U32 * (np.abs(W) @ np.abs(X)) + tiny), "z")
+    dx, _, _ = gpu.pw_conv_backward(dev(dz), dev(x), dev(w), want_dw=False, want_db=False)
+    check(host(dx), W.T @ D, (C_out + 2) * (U32 * (np.abs(W).T @ np.abs(D)) + tiny), "dx")
+    # the weight gradient of operands this far apart: dz of w's scale
+    dz = np.ldexp(data(13, N, C_in, C_out, HW)[3], ew).astype(np.float32)
+    D = dz.astype(np.float64)
+    _, dw, _ = gpu.pw_conv_backward(dev(dz), dev(x), dev(w), want_dx=False, want_db=False)
+    check(host(dw), np.einsum("nop,ncp->oc", D, X, optimize=True),
+          1026 * (U32 * np.einsum("nop,ncp->oc", np.abs(D), np.abs(X), optimize=True) + tiny), "dw")
 
 
 @pytest.mark.parametrize("value", [np.inf, -np.inf, np.nan, 3.4e38])
