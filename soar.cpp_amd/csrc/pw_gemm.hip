@@ -574,7 +574,7 @@ hipError_t launch_pw_gemm(const PwArgs& a, int64_t N, int64_t K, int64_t M, int6
             go(std::integral_constant<int, A() ? kGemmAccum : kGemmPlain>{}, F{}, std::true_type{});
         });
     } else if (accumulate) {
-        go(std::integral_constant<int, kGemmAccum>{}, F{}, F{});
+        return hipErrorInvalidValue;  // only input gradients are added
     } else {
         bsel(a.bias != nullptr, [&](auto B) {
             if (part)
