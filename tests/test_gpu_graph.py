@@ -77,11 +77,12 @@ def test_gn_silu_graph_replays(gpu, N, C, HW, G):
 
 CBA_CASES = [
     # (C_in, C_out, H, K): pointwise (K = 1) or depthwise CBA
-    (64, 64, 128, 1),    # MFMA conv, split K, statistics in the epilogue
+    (64, 64, 128, 1),    # block-tiled conv, statistics in the epilogue
+    (40, 64, 128, 1),    # MFMA conv, split K, statistics in the epilogue
     (32, 64, 16, 1),     # SIMT conv, then the one-launch GroupNorm
     (32, 32, 64, 7),     # depthwise k7 (multi-tile kernels), then GroupNorm
-    (256, 128, 64, 1),   # MFMA conv, K split over blocks (slices + reduce with statistics),
-                         # dx reading W in place
+    (256, 128, 64, 1),   # block-tiled conv; MFMA dx reading W in place
+    (512, 256, 32, 1),   # MFMA conv, K split over blocks (slices + reduce with statistics)
 ]
 
 

@@ -331,7 +331,40 @@ def torch_equal(a, b):
     return torch.equal(a, b)
 
 
-def test_misaligned_pointers_take_scalar_path(gpu, oracle):
+@pytest.mark.parametrize("HW,silu,residual,accumulate", [
+    (40000, True, False, False), (40001, True, True, True), (39998, False, True, False),
+    (40003, False, False, True)])
+def test_tensors_at_any_alignment(gpu, HW, silu, residual, accumulate):
+    """Every tensor one float past a 16-byte boundary: the bits of aligned
+    ones, and nothing written beside them."""
+    import torch
+    N, C, G = 1, 4, 2
+    g = torch.Generator(device="cuda").manual_seed(HW)
+    x, dy, dx0 = (torch.randn((N, C, HW), device="cuda", generator=g) for _ in range(3))
+    gamma, beta = torch.rand(C, device="cuda"), torch.randn(C, device="cuda")
+
+    def off(t):
+        buf = torch.full((t.numel() + 8,), 7.0, device="cuda")
+        buf[1:1 + t.numel()] = t.reshape(-1)
+        return buf, buf[1:1 + t.numel()].view(t.shape)
+
+    kw = dict(silu=silu, residual=residual)
+    y, st = gpu.gn_silu_forward(x, gamma, beta, G, eps=EPS, **kw)
+    want = gpu.gn_silu_backward(dy, x, gamma, beta, st, G, dx=dx0.clone(),
+                                accumulate_dx=accumulate, **kw)
+    ybuf, yo = off(torch.zeros_like(y))
+    _, st2 = gpu.gn_silu_forward(off(x)[1], gamma, beta, G, eps=EPS, y=yo, **kw)
+    dbuf, dxo = off(dx0)
+    got = gpu.gn_silu_backward(off(dy)[1], off(x)[1], gamma, beta, st2, G, dx=dxo,
+                               accumulate_dx=accumulate, **kw)
+    assert torch.equal(yo, y) and torch.equal(st2.mean, st.mean) and torch.equal(st2.rstd, st.rstd)
+    for a, b in zip(got, want):
+        assert torch.equal(a, b)
+    for buf in (ybuf, dbuf):
+        assert buf[0] == 7 and (buf[-7:] == 7).all()
+
+
+def test_misaligned_tensors_match_oracle(gpu, oracle):
     import torch
     N, C, HW, G = 1, 4, 40000, 2
     x, gamma, beta, dy = make_inputs(oracle, N, C, HW, G, "normal", 6)

@@ -38,6 +38,19 @@ def pw_path(request, gpu):
     gpu.tune(gpu.TUNE_PW_SPLITK, old_kz)
 
 
+def kernels(gpu, fn):
+    """The timer names of the launches of fn(), and its result."""
+    import torch
+    gpu.prof_summary()  # drop earlier records
+    gpu.prof_enable(True)
+    try:
+        out = fn()
+        torch.cuda.synchronize()
+        return {p["kernel"] for p in gpu.prof_summary()}, out
+    finally:
+        gpu.prof_enable(False)
+
+
 def rng_inputs(seed, N, C_in, C_out, HW, bias=True, kind="normal"):
     r = np.random.default_rng(seed)
     if kind == "offset":
@@ -109,9 +122,10 @@ FUSED_SHAPES = [
     (3, 16, 32, 1024, 8, "normal", True),      # exactly one chunk per plane
     # 300 pixel chunks of 1024: the streamed kernel's grid ends in a part-
     # filled window of the XCD-aware block order
-    (1, 64, 64, 300 * 1024, 16, "normal", True),
+    (1, 64, 40, 300 * 1024, 8, "normal", True),
+    (1, 64, 64, 300 * 1024, 16, "normal", True),   # block-tiled, two items a chunk
+    (1, 256, 128, 4096, 16, "normal", True),   # the Nano LKR at 1024^2, stride 16: block-tiled
     # small grids with K >= 128: K split over blocks (slices + reduce)
-    (1, 256, 128, 4096, 16, "normal", True),   # the Nano LKR at 1024^2, stride 16
     (1, 512, 256, 1024, 32, "offset", True),   # stride 32; large |mean|
     (1, 300, 72, 1000, 8, "normal", False),    # general path (C_in % 8), ragged HW
 ]
@@ -362,9 +376,9 @@ def test_pw_conv_backward_matches_oracle(gpu, oracle, pw_path, N, C_in, C_out, H
 
 WGRAD_WAVE_SHAPES = [
     # (N, C_in, C_out, HW)
-    (1, 64, 64, 65536),     # one 64 x 64 tile, 1024 wave chunks of 64 pixels
+    (1, 64, 40, 65536),     # one 64 x 64 tile, 1024 wave chunks of 64 pixels
     (3, 24, 8, 333),        # one block per plane: 11 steps over up to 8 waves
-    (1, 130, 72, 4096),     # 6 partial tiles, ragged rows and columns
+    (1, 130, 40, 4096),     # 3 partial tiles, ragged rows and columns
     (2, 32, 48, 2500),      # 32-column tiles; the last block of a plane is short
 ]
 
@@ -391,7 +405,9 @@ def test_pw_wgrad_waves_per_block(gpu, oracle, restore_pw_small, N, C_in, C_out,
             gpu.tune(gpu.TUNE_PW_WG_WAVES, waves)
             runs = []
             for _ in range(2):
-                _, dw, db = gpu.pw_conv_backward(dzd, xd, wd, want_dx=False)
+                names, (_, dw, db) = kernels(gpu, lambda: gpu.pw_conv_backward(dzd, xd, wd,
+                                                                               want_dx=False))
+                assert "pw_conv_wgrad" in names, names
                 runs.append((host(dw), host(db)))
             for got, t, bnd, name in ((runs[0][0], tw, bw, "dw"), (runs[0][1], tb, bb, "db")):
                 err = np.abs(got.astype(np.float64).reshape(-1) - t)
@@ -401,6 +417,32 @@ def test_pw_wgrad_waves_per_block(gpu, oracle, restore_pw_small, N, C_in, C_out,
             assert np.array_equal(runs[0][0], runs[1][0]) and np.array_equal(runs[0][1], runs[1][1])
     finally:
         gpu.tune(gpu.TUNE_PW_WG_WAVES, old)
+
+
+@pytest.mark.parametrize("waves", [1, 2, 4, 8])
+def test_pw_wgrad_wide_ragged(gpu, waves):
+    """The MFMA weight gradient of a wide layer, which runs above 2^18 pixels
+    only: 2 x 3 tiles of 64 x 64, the last of each ragged, and a ragged last
+    step, against float64 products on the device."""
+    import torch
+    C_in, C_out, HW = 130, 72, 2 ** 18 + 5
+    old = gpu.tune_get(gpu.TUNE_PW_WG_WAVES)
+    g = torch.Generator(device="cuda").manual_seed(9)
+    dz = torch.randn((1, C_out, HW), device="cuda", generator=g)
+    x = torch.randn((1, C_in, HW), device="cuda", generator=g)
+    w = torch.zeros((C_out, C_in), device="cuda")
+    gpu.tune(gpu.TUNE_PW_WG_WAVES, waves)
+    try:
+        names, (_, dw, db) = kernels(gpu, lambda: gpu.pw_conv_backward(dz, x, w, want_dx=False))
+    finally:
+        gpu.tune(gpu.TUNE_PW_WG_WAVES, old)
+    assert "pw_conv_wgrad" in names, names
+    a, b = dz[0].double(), x[0].double()
+    # fp32 sums over a wave's chunk (6 tiles HW / 2048 pixels, at most 800) and
+    # up to 8 waves, then float64
+    bound = (800 + 8 + 2) * U32
+    assert ((dw.double() - a @ b.T).abs() <= bound * (a.abs() @ b.abs().T)).all()
+    assert ((db.double() - a.sum(1)).abs() <= bound * a.abs().sum(1)).all()
 
 
 @pytest.mark.parametrize("C_in,C_out,HW", [(32, 32, 1000), (128, 256, 2048)])
@@ -603,9 +645,11 @@ def test_pw_small_planes_match_oracle(gpu, oracle, restore_pw_small, N, C_in, C_
 DETERMINISM_CASES = [
     # (N, C_in, C_out, HW, limit): which path runs
     (1, 256, 512, 16, None),        # SIMT forward / dx / weight gradient (K split over waves)
-    (1, 256, 128, 4096, None),      # MFMA small grid: K over 4 blocks x 4 waves, slice reduce
+    (1, 512, 256, 1024, None),      # MFMA small grid: K over 4 blocks x 4 waves, slice reduce
                                     # with the statistics; dx K over the waves of a block
-    (1, 64, 64, 262144, None),      # MFMA, two K steps in flight (large grid)
+    (1, 64, 40, 262144, None),      # MFMA, streamed (large grid)
+    (1, 256, 128, 4096, None),      # block-tiled
+    (1, 64, 64, 262144, None),      # block-tiled, several items a chunk
     (3, 24, 40, 1000, 0),           # MFMA forced, general shapes
 ]
 

@@ -11,6 +11,7 @@ import numpy as np
 import pytest
 
 from test_gpu_parity import EPS, assert_stats, assert_vals, dev, host
+from test_gpu_pw_conv import kernels
 
 pytestmark = pytest.mark.gpu
 
@@ -23,9 +24,22 @@ SHAPES = [
     (2, 51, 130, 2055),    # three row tiles, HW % 4 = 3
     (1, 64, 64, 4098),     # whole row tile, a pixel tile of 2
     (1, 160, 200, 4100),   # five K steps, two ci tiles in the weight gradient
-    (1, 132, 256, 1025),   # K % 32 = 4; a pixel tile of one pixel
+    (1, 132, 256, 2817),   # K % 32 = 4; a pixel tile of one pixel
     (5, 128, 72, 1000),    # several samples, ragged rows
+    # chunks of 384 and 136 pixels: items of 128, 128, 128 | 128, 8 in a block,
+    # four row tiles, the last of 8 rows
+    (256, 200, 200, 520),
 ]
+
+
+@pytest.fixture(autouse=True)
+def no_simt(gpu, request):
+    """The block-tiled kernels also where k_pw_small would run."""
+    old = gpu.tune_get(gpu.TUNE_PW_SMALL)
+    if "leaves_small" not in request.node.name:
+        gpu.tune(gpu.TUNE_PW_SMALL, 0)
+    yield
+    gpu.tune(gpu.TUNE_PW_SMALL, old)
 
 
 def data(seed, N, C_in, C_out, HW):
@@ -48,13 +62,16 @@ def test_pw_gemm_matches_float64(gpu, oracle, shape):
     x, w, b, dz = data(7, *shape)
     X, W, D = x.astype(np.float64), w.astype(np.float64), dz.astype(np.float64)
     dzd, xd, wd = dev(dz), dev(x), dev(w)
-    z = gpu.pw_conv_forward(xd, wd, dev(b))
+    names, z = kernels(gpu, lambda: gpu.pw_conv_forward(xd, wd, dev(b)))
+    assert "pw_conv_tiled" in names, names
     zb = (C_in + 2) * U32 * (np.abs(W) @ np.abs(X) + np.abs(b)[:, None])
     check(host(z), W @ X + b[:, None], zb, "z")
 
     G = 1 if C_out % 2 else 2
     gamma, beta = np.linspace(0.5, 1.5, C_out, dtype=np.float32), np.zeros(C_out, np.float32)
-    z2, y, st = gpu.pw_conv_gn_silu_forward(xd, wd, dev(b), dev(gamma), dev(beta), G, eps=EPS)
+    names, (z2, y, st) = kernels(gpu, lambda: gpu.pw_conv_gn_silu_forward(
+        xd, wd, dev(b), dev(gamma), dev(beta), G, eps=EPS))
+    assert "pw_conv_gn_stats_tiled" in names, names
     check(host(z2), W @ X + b[:, None], zb, "z with statistics")
     ty, tm, tr = oracle.gn_silu_fwd_f64(host(z2), gamma, beta, N, C_out, HW, G, EPS)
     assert_vals(host(y), ty, "y")
@@ -62,7 +79,9 @@ def test_pw_gemm_matches_float64(gpu, oracle, shape):
 
     old = np.linspace(-1.0, 1.0, N * C_in * HW, dtype=np.float32).reshape(N, C_in, HW)
     for acc in (False, True):
-        dx_, dw_, db_ = gpu.pw_conv_backward(dzd, xd, wd, dx=dev(old), accumulate_dx=acc)
+        names, (dx_, dw_, db_) = kernels(gpu, lambda: gpu.pw_conv_backward(
+            dzd, xd, wd, dx=dev(old), accumulate_dx=acc))
+        assert {"pw_conv_dgrad_tiled", "pw_conv_wgrad_tiled"} <= names, names
         bx = (C_out + 3) * U32 * (np.abs(W).T @ np.abs(D) + np.abs(old))
         check(host(dx_), W.T @ D + (old if acc else 0.0), bx, "dx")
     tw = np.einsum("nop,ncp->oc", D, X, optimize=True)
@@ -111,6 +130,15 @@ def test_pw_gemm_non_finite_operands(gpu, value):
         z = host(gpu.pw_conv_forward(dev(x), dev(w)))
         want = w @ x[0, :, 777]
         np.testing.assert_allclose(z[0, :, 777], want, rtol=1e-5)
+        # with the statistics: the same z, and groups that it does not reach
+        G = 8
+        z2, y, st = gpu.pw_conv_gn_silu_forward(dev(x), dev(w), None,
+                                                dev(np.ones(C_out, np.float32)),
+                                                dev(np.zeros(C_out, np.float32)), G, eps=EPS)
+        np.testing.assert_array_equal(host(z2), z)
+        reached = (~np.isfinite(z[0])).any(1).reshape(G, -1).any(1)
+        assert np.array_equal(np.isnan(host(st.mean)) | np.isinf(host(st.mean)), reached)
+        assert np.isfinite(host(y)[0][~np.repeat(reached, C_out // G)]).all()
         keep = np.arange(HW) != 777
         np.testing.assert_allclose(z[0][4:70, keep], clean[0][4:70, keep], rtol=1e-4, atol=1e-4)
         dx, dw, _ = gpu.pw_conv_backward(dev(dz), dev(x), dev(w))
@@ -146,18 +174,9 @@ def test_pw_gemm_leaves_small_layers(gpu, shape, forward, fused, dgrad):
     N, C_in, C_out, HW = shape
     x, w, b, dz = (dev(v) for v in data(5, *shape))
     ga, be = torch.ones(C_out, device="cuda"), torch.zeros(C_out, device="cuda")
-
-    def kernels(fn):
-        gpu.prof_summary()  # drop earlier records
-        gpu.prof_enable(True)
-        fn()
-        torch.cuda.synchronize()
-        names = {p["kernel"] for p in gpu.prof_summary()}
-        gpu.prof_enable(False)
-        return names
-
-    assert ("pw_conv_tiled" in kernels(lambda: gpu.pw_conv_forward(x, w, b))) == forward
-    got = kernels(lambda: gpu.pw_conv_gn_silu_forward(x, w, b, ga, be, 8))
+    got, _ = kernels(gpu, lambda: gpu.pw_conv_forward(x, w, b))
+    assert ("pw_conv_tiled" in got) == forward, got
+    got, _ = kernels(gpu, lambda: gpu.pw_conv_gn_silu_forward(x, w, b, ga, be, 8))
     assert ("pw_conv_gn_stats_tiled" in got) == fused, got
-    got = kernels(lambda: gpu.pw_conv_backward(dz, x, w, want_dw=False, want_db=False))
+    got, _ = kernels(gpu, lambda: gpu.pw_conv_backward(dz, x, w, want_dw=False, want_db=False))
     assert ("pw_conv_dgrad_tiled" in got) == dgrad, got
