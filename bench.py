@@ -8,6 +8,10 @@ through the C-ABI of libsoar_gn.so on one GPU.  Prints one JSON line:
 
   value      algorithmic HBM bytes of the step (8 tensor passes: fwd 3T,
              bwd 5T, T = N*C*H*W*4) / measured step time, in GB/s;
+  frac_of_peak  the share of the HBM peak, of the bytes that the step's
+             kernels move (null without kernel timing): a kernel that keeps
+             a unit on chip between its passes moves fewer than `value`
+             counts;
   roofline   the dominant kernel's algorithmic bytes per launch / its mean
              hipEvent-timed duration over the timed region, against the
              8 TB/s HBM peak; `traffic` is the rocprofv3-measured bytes per
@@ -868,6 +872,9 @@ def main():
     kernels = [] if args.no_kernel_timing else timed(True)[2]
     alg = step.algorithmic_bytes()
     value = alg / (ms * 1e-3) / 1e9
+    moved = alg if hasattr(step, "kernel_bytes") else None
+    if kernels and moved is None:
+        moved = sum(PASSES.get(k["kernel"], 0) for k in kernels) * step.T * len(step.params)
 
     roofline = None
     kinfo = {}
@@ -944,7 +951,7 @@ def main():
                "N": N, "C": C, "H": int(HW ** 0.5), "W": int(HW ** 0.5), "G": G,
                "eps": 1e-5, "blocks": blocks, "residual": residual,
                **({"C_in": CBA_C_IN} if args.config.startswith("cba_pw") else {}),
-               "algorithmic_bytes_per_step": alg}
+               "algorithmic_bytes_per_step": alg, "moved_bytes_per_step": moved}
     if tuning:
         cfg["tuning"] = tuning
     out = {
@@ -961,7 +968,7 @@ def main():
         "dtype": "fp32",
         "data": data,
         "config": cfg,
-        "frac_of_peak": round(value / PEAK_GBS, 4),
+        "frac_of_peak": round(moved / (ms * 1e-3) / 1e9 / PEAK_GBS, 4) if moved else None,
         "wall_s_timed": round(wall, 4),
         "roofline": roofline,
         "kernels": kinfo,
