@@ -214,9 +214,12 @@ SOAR_API int soar_zero3(float* a, size_t na, float* b, size_t nb, float* c,
 /* ---- pointwise convolution, the producer of CBA's GroupNorm ---------- */
 /* The 1x1 / stride 1 / no-padding / groups 1 convolution of CBA blocks
  * (Down.pw, LKR.pw1/pw2, Ctx.cv1/cv2; src/nn/blocks.cpp:429-480) is a GEMM
- * over the pixel axis; it runs on the fp32 matrix cores (v_mfma_f32_32x32x2
- * f32: fp32 products, fp32 accumulation).  weight is [C_out][C_in], bias
- * [C_out] or NULL; activations are [C][HW] per sample. */
+ * over the pixel axis, with the error of fp32 products and sums: small ones
+ * run on the vector units, layers of 48 rows and channels and more on the
+ * bf16 matrix cores with every operand split into three bf16 parts (24 bits,
+ * any magnitude), the others on the fp32 matrix cores (v_mfma_f32_32x32x2
+ * f32).  weight is [C_out][C_in], bias [C_out] or NULL; activations are
+ * [C][HW] per sample. */
 
 /* out[co][p] = bias[co] + sum_ci weight[co][ci] * in[ci][p], one sample.
  * Replaces: conv2d_1x1_forward (cuda_kernels.hpp:57-58,

@@ -19,10 +19,12 @@
 // three blocks share a CU, and one block's loads, splits and waits run
 // beside another's MFMAs.  What bounds a large grid is the LDS traffic (9
 // KB read per 12 MFMAs of a wave, beside the staging) and the MFMAs
-// together: 150-160 TFLOP/s of fp32 product, 104 before.  (Measured and not
-// kept, us for the forward / input gradient / weight gradient of 192 -> 384
-// channels at 128^2 pixels, 23.9 / 26.5 / 26.0 as it is: 128 x 128 tiles 26.7
-// / 30.4 / 37; loads two steps ahead 28.3 / 28.3 / 27.7; two stages with the
+// together: 130 TFLOP/s of fp32 product for the input gradient of 128 -> 256
+// channels over 2^20 pixels (k_pw_conv 92), 96 / 87 / 89 for 192 -> 384 at
+// 128^2 (25.3 / 27.8 / 27.1 us forward with statistics / input gradient /
+// weight gradient).  (Measured and not kept, before the operands' scale, us
+// for those three, 23.9 / 26.5 / 26.0 as it was: 128 x 128 tiles 26.7 / 30.4
+// / 37; loads two steps ahead 28.3 / 28.3 / 27.7; two stages with the
 // next step's splits between the MFMAs, two blocks per CU, 30.6 / 29.9 / 35.7.)
 //
 // Operands whose K axis runs along the rows (W in the forward, dz and x in
