@@ -183,8 +183,8 @@ def test_team_on_two_streams(gpu):
 @pytest.mark.parametrize("backward", [False, True])
 def test_streams_cost_no_more_than_two_launches(gpu, wait_us, shape, backward):
     """Two streams' calls at once take no longer than where every call reads
-    its tensor twice (bar: a third more, for timing).  Where a team needed more
-    than half of the chip, both streams' teams stood in each other's way: 2 to
+    its tensor twice (bar: half more, for timing).  Where a team needed more
+    than half of the chip, both streams' teams stood in each other's way: 3.7 to
     20 times as long."""
     N, C, HW, G = shape
     calls = []
@@ -221,4 +221,4 @@ def test_streams_cost_no_more_than_two_launches(gpu, wait_us, shape, backward):
         wait_us(wait)
         t = run()
         best[wait] = min(t, best.get(wait, t))
-    assert best[default] <= 1.33 * best[-1], best
+    assert best[default] <= 1.5 * best[-1], best
