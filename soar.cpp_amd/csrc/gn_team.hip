@@ -193,10 +193,11 @@ __device__ __forceinline__ void store_vec(f4 o, float* __restrict__ y, const Tea
 }
 
 // The value of slot `it` once it is set; false when the limit passes first or
-// another block of the call has left (wave-uniform).  A wait costs one round trip past the caches per look.  (With
-// a slot per chunk, 2048 per 64 MB unit, the looks of 256 blocks were 19 MB
-// each and a unit waited 7 us.  16-byte loads with the scope bits of a
-// volatile buffer load, sc0 sc1, kept returning old words; these are sc1.)
+// another block of the call has left (wave-uniform).  A wait costs one round
+// trip past the caches per look.  (With a slot per chunk, 2048 per 64 MB unit,
+// the looks of 256 blocks were 19 MB each and a unit waited 7 us.  16-byte
+// loads with the scope bits of a volatile buffer load, sc0 sc1, kept returning
+// old words; these are sc1.)
 __device__ __forceinline__ bool poll(double2& v, const u64* __restrict__ slots, int it,
                                      const Team& g, const TeamWs& w, u64 t0) {
     const u64* s = slots + 2 * min(it, g.items - 1);

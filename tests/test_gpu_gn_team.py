@@ -127,7 +127,12 @@ def test_team_leaves_overlapping_outputs_alone(gpu):
     assert (d - dx).abs().max() <= 4 * 2.0 ** -23 * dx.abs().max()
 
 
-def test_team_graph_replays(gpu):
+@pytest.mark.parametrize("wait", [None, 0, -2])
+def test_team_graph_replays(gpu, wait_us, wait):
+    """Replays with other work between them, also where blocks leave their
+    shares to the launch after."""
+    if wait is not None:
+        wait_us(wait)
     x, dy, gamma, beta = tensors(3, 64, 65536, True)
     ws = gpu.workspace(3, 64, 65536, 8)
     want = both(gpu, x, dy, gamma, beta, 8, True, False)
